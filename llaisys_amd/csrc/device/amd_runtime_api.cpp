@@ -191,6 +191,25 @@ void raiseIfError(llaisysStream_t s) {
     if (code != 0) LLAISYS_FAIL(std::runtime_error, "device error code " << code, "device error");
 }
 
+namespace {
+// Moves the slot to a buffer of at least `bytes`, zeroed (kernels that keep a completion counter
+// in the workspace expect it zeroed once).  The old buffer is freed, after a device
+// synchronisation, once no graph holds it.
+int growWorkspace(std::shared_ptr<WsBuffer> &cur, size_t bytes, const char *&what) {
+    const size_t n = bytes < (size_t(1) << 20) ? (size_t(1) << 20) : bytes;
+    void *p = nullptr;
+    what = "hipMalloc(workspace)";
+    if (const int st = hipMalloc(&p, n)) return st;
+    what = "hipMemset(workspace)";
+    if (const int st = hipMemset(p, 0, n)) {
+        (void)hipFree(p);
+        return st;
+    }
+    cur = std::make_shared<WsBuffer>(p, n);
+    return hipSuccess;
+}
+} // namespace
+
 void *workspace(int dev, size_t bytes) {
     CHECK_ARGUMENT(dev >= 0 && dev < kMaxDevices, "device id out of range");
     WsSlots &ws = wsSlots();
@@ -204,17 +223,26 @@ void *workspace(int dev, size_t bytes) {
                              << " bytes during HIP graph capture; set LLAISYS_GRAPH_WORKSPACE_BYTES "
                                 "above that before llaisysGraphBeginCapture",
                          "workspace growth during capture");
-        size_t n = bytes < (size_t(1) << 20) ? (size_t(1) << 20) : bytes;
-        void *p = nullptr;
-        check(hipMalloc(&p, n), "hipMalloc(workspace)");
-        // Kernels that keep a completion counter in the workspace expect it zeroed once.
-        const int st = hipMemset(p, 0, n);
-        if (st != hipSuccess) {
-            (void)hipFree(p);
-            check(st, "hipMemset(workspace)");
-        }
-        // The old buffer is freed (after a device synchronisation) once no graph holds it.
-        cur = std::make_shared<WsBuffer>(p, n);
+        const char *what = nullptr;
+        const int st = growWorkspace(cur, bytes, what);
+        check(st, what);
+    }
+    return cur->ptr;
+}
+
+void *tryWorkspace(int dev, size_t bytes, llaisysStream_t s) {
+    CHECK_ARGUMENT(dev >= 0 && dev < kMaxDevices, "device id out of range");
+    WsSlots &ws = wsSlots();
+    std::shared_ptr<WsBuffer> &cur = ws.buf[dev];
+    if (cur && cur->size >= bytes) return cur->ptr;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (ws.capturing[dev] || hipStreamIsCapturing(static_cast<hipStream_t>(s), &cap) != hipSuccess ||
+        cap != hipStreamCaptureStatusNone)
+        return nullptr;
+    const char *what = nullptr;
+    if (growWorkspace(cur, bytes, what) != hipSuccess) {
+        (void)hipGetLastError(); // the caller goes on without: leave no sticky error
+        return nullptr;
     }
     return cur->ptr;
 }

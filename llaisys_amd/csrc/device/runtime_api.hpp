@@ -29,6 +29,10 @@ void raiseIfError(llaisysStream_t stream);
 // least `bytes` of device memory, zeroed when first allocated.  A growth moves the thread
 // to a new buffer; the old one is freed once no captured graph holds it.
 void *workspace(int device_id, size_t bytes);
+// The same scratch for a caller that can do without: null where it would have to grow while
+// `stream` is being captured (by llaisysGraphBeginCapture or by the caller itself), or where the
+// memory is not there.
+void *tryWorkspace(int device_id, size_t bytes, llaisysStream_t stream);
 
 // HIP-graph capture of the work enqueued on `stream` (the current device's context stream).
 // beginCapture reserves the workspace a captured op may need (growth during capture is an

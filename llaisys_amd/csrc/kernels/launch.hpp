@@ -119,12 +119,27 @@ void selfAttention(void *out, const void *q, const void *k, const void *v, const
                    size_t d, size_t dv, float scale, llaisysDataType_t dt, void *ws,
                    size_t ws_bytes, hipStream_t stream);
 
-// out [rows, N] = x [rows, K] w^T (+ bias [N]); with w_scale non-null w is INT8 codes
-// [N, K] and the sum of each output channel n is multiplied by w_scale[n] (W8A16).  rows,
-// K and N below 2^31.
-void linear(void *out, const void *x, const void *w, const float *w_scale, const void *bias,
-            size_t rows, size_t in_features, size_t out_features, llaisysDataType_t dt,
-            hipStream_t stream);
+// out [rows, N] = x [rows, K] w^T (+ bias), w of N rows; with `scale` non-null w is INT8 codes and
+// the sum of each weight row n is multiplied by scale[n] (W8A16).  With `swiglu` w, scale and bias
+// have 2 N rows, the gate's first, and out = swiglu(gate, up), both rounded to the element type.
+// rows, K and the weight rows are below 2^31.
+struct LinearCall {
+    void *out;
+    const void *x;
+    const void *w;
+    const float *scale;
+    const void *bias;
+    size_t rows, K, N;
+    bool swiglu;
+    llaisysDataType_t dt;
+};
+// Workspace that lets `linear` split K over blocks as it would like to; with less (or none) it
+// runs without splitting.
+size_t linearWorkspaceBytes(const LinearCall &c);
+void linear(const LinearCall &c, void *ws, size_t ws_bytes, hipStream_t stream);
+// Whether `linear` takes c with swiglu in one call (else: two calls on the weight's halves, then
+// swiglu, which gives the same values).
+bool linearSwigluFused(const LinearCall &c);
 
 // One row: h = residual ? T(in + residual) : in (h stored to residual_out when residual is
 // non-null), xn = rms_norm(h) as rmsNorm computes it, y = linear(xn) (W8A16 when w_scale is

@@ -24,13 +24,15 @@
 //    weights or other K) stages them through registers and a padded LDS tile, converting
 //    INT8 codes to exact bf16 / f16 on the way.  Blocks map to the 8 XCDs so that a weight
 //    tile stays in one L2 while the row tiles pass over it.
-//  - anything else (f32, unaligned rows, K not a multiple of 8 / 16): linearScalar, one
-//    thread per output with the reference's sequential sum.
+//  - f32: linearGemvRow / linearGemv for one row, linear_gemm.hip for more (K % 4 == 0).
+//  - anything else (unaligned rows, K not a multiple of a 16-byte chunk, f32 against INT8
+//    weights): linearScalar, one thread per output with the reference's sequential sum.
 // INT8 codes enter every MFMA as exact bf16 / f16 values and the per-channel scale multiplies
 // the f32 sum once.
 #include "common.hpp"
 #include "launch.hpp"
 #include "linear_common.hpp"
+#include "linear_gemm.hpp"
 #include "rowplan.hpp"
 
 #include <algorithm>
@@ -370,20 +372,22 @@ __global__ void __launch_bounds__(1024)
 template <typename T, bool kInt8, int M>
 __global__ void __launch_bounds__(256)
     linearGemv(LinearArgs a) {
-    constexpr int E = kInt8 ? 16 : 8;  // weight elements per 16-byte chunk
-    constexpr int U = 4;               // chunks in flight per lane
+    using F = Fmt<T>;
+    constexpr int E = kInt8 ? 16 : F::kVec;  // weight elements per 16-byte chunk
+    constexpr int XH = E / F::kVec;          // 16-byte chunks of x beside it
+    constexpr int U = 4;                     // chunks in flight per lane
     const int lane = int(threadIdx.x) % kWave;
     const int n = int(blockIdx.x) * 4 + int(threadIdx.x) / kWave; // wave-uniform
     if (n >= a.N) return;
     const int nc = a.K / E; // K % E == 0
-    const char *wrow = static_cast<const char *>(a.w) + size_t(n) * a.K * (kInt8 ? 1 : 2);
+    const char *wrow = static_cast<const char *>(a.w) + size_t(n) * a.K * (kInt8 ? 1 : F::kBytes);
     const char *xb = static_cast<const char *>(a.x);
     float acc[M];
 #pragma unroll
     for (int m = 0; m < M; ++m) acc[m] = 0.0f;
     for (int c0 = lane; c0 < nc; c0 += kWave * U) {
         // all loads first (a chunk past the row end reads chunk 0 and is masked below)
-        v4u wv[U], xv[U][M][E / 8];
+        v4u wv[U], xv[U][M][XH];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int c = c0 + kWave * u < nc ? c0 + kWave * u : 0;
@@ -391,8 +395,8 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
             for (int m = 0; m < M; ++m)
 #pragma unroll
-                for (int h = 0; h < E / 8; ++h)
-                    xv[u][m][h] = *reinterpret_cast<const v4u *>(xb + (size_t(m) * a.K + size_t(c) * E + 8 * h) * 2);
+                for (int h = 0; h < XH; ++h)
+                    xv[u][m][h] = load16<T>(xb, size_t(m) * a.K + size_t(c) * E + F::kVec * h);
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -408,11 +412,11 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
             for (int m = 0; m < M; ++m)
 #pragma unroll
-                for (int h = 0; h < E / 8; ++h) {
-                    float xf[8];
-                    Fmt<T>::unpack(xv[u][m][h], xf);
+                for (int h = 0; h < XH; ++h) {
+                    float xf[F::kVec];
+                    F::unpack(xv[u][m][h], xf);
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) acc[m] = __builtin_fmaf(xf[e], wf[8 * h + e], acc[m]);
+                    for (int e = 0; e < F::kVec; ++e) acc[m] = __builtin_fmaf(xf[e], wf[F::kVec * h + e], acc[m]);
                 }
         }
     }
@@ -442,9 +446,9 @@ template <typename T, bool kInt8, int J, int C, bool kLds, int NW>
 __global__ void __launch_bounds__(NW * kWave)
     linearGemvRow(LinearArgs a) {
     using F = Fmt<T>;
-    constexpr int E = kInt8 ? 16 : 8; // weight elements per 16-byte chunk
+    constexpr int E = kInt8 ? 16 : F::kVec; // weight elements per 16-byte chunk
     extern __shared__ __align__(16) char xs_raw[];
-    const uint16_t *xs = kLds ? reinterpret_cast<const uint16_t *>(xs_raw) : static_cast<const uint16_t *>(a.x);
+    const char *xs = kLds ? xs_raw : static_cast<const char *>(a.x);
     const int lane = int(threadIdx.x) % kWave;
     const int n0 = (int(blockIdx.x) * NW + int(threadIdx.x) / kWave) * C; // wave-uniform
     const int nc = a.K / E;
@@ -454,7 +458,7 @@ __global__ void __launch_bounds__(NW * kWave)
 #pragma unroll
     for (int ci = 0; ci < C; ++ci) {
         const int n = n0 + ci;
-        const char *wrow = static_cast<const char *>(a.w) + size_t(n < a.N ? n : a.N - 1) * a.K * (kInt8 ? 1 : 2);
+        const char *wrow = static_cast<const char *>(a.w) + size_t(n < a.N ? n : a.N - 1) * a.K * (kInt8 ? 1 : F::kBytes);
 #pragma unroll
         for (int j = 0; j < J; ++j) {
             const int c = lane + kWave * j;
@@ -462,7 +466,7 @@ __global__ void __launch_bounds__(NW * kWave)
         }
     }
     if constexpr (kLds) {
-        for (int i = int(threadIdx.x); i < a.K / 8; i += NW * kWave)
+        for (int i = int(threadIdx.x); i < a.K / F::kVec; i += NW * kWave)
             reinterpret_cast<v4u *>(xs_raw)[i] = reinterpret_cast<const v4u *>(a.x)[i];
         __syncthreads();
     }
@@ -477,7 +481,7 @@ __global__ void __launch_bounds__(NW * kWave)
         if (c >= nc) continue; // (the lane's remaining chunks are past the end too)
         float xf[E];
 #pragma unroll
-        for (int h = 0; h < E / 8; ++h) F::unpack(*reinterpret_cast<const v4u *>(xs + c * E + 8 * h), xf + 8 * h);
+        for (int h = 0; h < E / F::kVec; ++h) F::unpack(load16<T>(xs, c * E + F::kVec * h), xf + F::kVec * h);
 #pragma unroll
         for (int ci = 0; ci < C; ++ci) {
             float wf[E];
@@ -541,7 +545,7 @@ bool launchRowJ(const LinearArgs &a, int j, hipStream_t s) {
     if constexpr (J > 0) {
         if (j == J) {
             const unsigned blocks = unsigned((a.N + NW * C - 1) / (NW * C));
-            linearGemvRow<T, kInt8, J, C, kLds, NW><<<blocks, NW * kWave, kLds ? size_t(a.K) * 2 : 0, s>>>(a);
+            linearGemvRow<T, kInt8, J, C, kLds, NW><<<blocks, NW * kWave, kLds ? size_t(a.K) * Fmt<T>::kBytes : 0, s>>>(a);
             return true;
         }
         return launchRowJ<T, kInt8, C, kLds, NW, J - 1>(a, j, s);
@@ -551,8 +555,8 @@ bool launchRowJ(const LinearArgs &a, int j, hipStream_t s) {
 
 template <typename T, bool kInt8>
 bool launchGemv1(const LinearArgs &a, hipStream_t s) {
-    constexpr int E = kInt8 ? 16 : 8;
-    if (a.K % E != 0 || size_t(a.K) * 2 > 64 * 1024) return false;
+    constexpr int E = kInt8 ? 16 : Fmt<T>::kVec;
+    if (a.K % E != 0 || size_t(a.K) * Fmt<T>::kBytes > 64 * 1024) return false;
     const int j = (a.K / E + kWave - 1) / kWave;
     if (j < 1 || j > 24) return false;
     if constexpr (kInt8) {
@@ -621,6 +625,14 @@ void launch(const LinearArgs &a, hipStream_t s) {
         }
         return;
     }
+    // f32, one row: the same GEMV (several rows: linear_gemm.hip)
+    if constexpr (std::is_same_v<T, F32> && !kInt8) {
+        if (a.M == 1 && a.K > 0 && a.K % 4 == 0 && al(a.x, 16) && al(a.w, 16)) {
+            if (launchGemv1<F32, false>(a, s)) return;
+            linearGemv<F32, false, 1><<<unsigned((a.N + 3) / 4), 256, 0, s>>>(a);
+            return;
+        }
+    }
     const size_t n = size_t(a.M) * a.N;
     linearScalar<T, kInt8><<<unsigned((n + 255) / 256), 256, 0, s>>>(a);
 }
@@ -637,14 +649,17 @@ void dispatch(const LinearArgs &a, llaisysDataType_t dt, hipStream_t s) {
 
 } // namespace
 
-void linear(void *out, const void *x, const void *w, const float *w_scale, const void *bias,
-            size_t rows, size_t in_features, size_t out_features, llaisysDataType_t dt,
-            hipStream_t s) {
-    const LinearArgs a{out, x, w, w_scale, bias, int(rows), int(out_features), int(in_features)};
-    if (w_scale)
-        dispatch<true>(a, dt, s);
+bool linearSwigluFused(const LinearCall &c) { return gemmTakes(c); }
+
+size_t linearWorkspaceBytes(const LinearCall &c) { return gemmTakes(c) ? gemmWorkspaceBytes(c) : 0; }
+
+void linear(const LinearCall &c, void *ws, size_t ws_bytes, hipStream_t s) {
+    if (gemmTakes(c)) return gemm(c, ws, ws_bytes, s);
+    const LinearArgs a{c.out, c.x, c.w, c.scale, c.bias, int(c.rows), int(c.N), int(c.K)};
+    if (c.scale)
+        dispatch<true>(a, c.dt, s);
     else
-        dispatch<false>(a, dt, s);
+        dispatch<false>(a, c.dt, s);
 }
 
 } // namespace llaisys::kernels

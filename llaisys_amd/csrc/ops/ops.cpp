@@ -508,6 +508,22 @@ size_t checkLinear(const tensor_t &out, const tensor_t &in, const tensor_t &weig
            "Linear: dimensions must be below 2^31");
     return rows;
 }
+
+// The library scratch past its reserved head, with `head` bytes the call needs and, where the
+// scratch can hold them, up to `want` more for the linear's split sums (`spare` bytes of them).
+char *linearScratch(int dev, size_t head, size_t want, size_t &spare, hipStream_t s) {
+    head += kernels::kScratchReserved;
+    void *ws = want ? device::amd::tryWorkspace(dev, head + want, s) : nullptr;
+    spare = ws ? want : 0;
+    if (!ws && head > kernels::kScratchReserved) ws = device::amd::workspace(dev, head);
+    return ws ? static_cast<char *>(ws) + kernels::kScratchReserved : nullptr;
+}
+
+void runLinear(const kernels::LinearCall &c, int dev, hipStream_t s) {
+    size_t spare = 0;
+    char *ws = linearScratch(dev, 0, kernels::linearWorkspaceBytes(c), spare, s);
+    kernels::linear(c, ws, spare, s);
+}
 } // namespace
 
 // reference src/ops/linear/op.cpp:10-42
@@ -523,9 +539,9 @@ void linear(tensor_t out, tensor_t in, tensor_t weight, tensor_t bias) {
     const size_t rows = checkLinear(out, in, weight, bias, has_bias);
     requireFloat(in->dtype());
     auto s = streamFor(in);
-    kernels::linear(out->data(), in->data(), weight->data(), nullptr,
-                    has_bias ? bias->data() : nullptr, rows, weight->shape()[1],
-                    weight->shape()[0], in->dtype(), s);
+    runLinear({out->data(), in->data(), weight->data(), nullptr, has_bias ? bias->data() : nullptr, rows,
+               weight->shape()[1], weight->shape()[0], false, in->dtype()},
+              in->deviceId(), s);
     launched("linear");
 }
 
@@ -546,10 +562,10 @@ void linearW8A16(tensor_t out, tensor_t in, tensor_t w_codes, tensor_t w_scale, 
            "LinearW8A16: one contiguous scale per output feature");
     requireFloat(in->dtype());
     auto s = streamFor(in);
-    kernels::linear(out->data(), in->data(), w_codes->data(),
-                    reinterpret_cast<const float *>(w_scale->data()),
-                    has_bias ? bias->data() : nullptr, rows, w_codes->shape()[1],
-                    w_codes->shape()[0], in->dtype(), s);
+    runLinear({out->data(), in->data(), w_codes->data(), reinterpret_cast<const float *>(w_scale->data()),
+               has_bias ? bias->data() : nullptr, rows, w_codes->shape()[1], w_codes->shape()[0], false,
+               in->dtype()},
+              in->deviceId(), s);
     launched("linearW8A16");
 }
 
@@ -632,23 +648,29 @@ void rmsNormLinear(tensor_t out, tensor_t residual_out, tensor_t in, tensor_t re
         launched("rmsNormLinear");
         return;
     }
-    // The same ops one after another through library scratch: xn [rows, K], then (swiglu)
-    // gate and up [rows, N] from the two halves of the weight.
+    // The same ops one after another through library scratch: xn [rows, K], then the linear,
+    // with swiglu in its epilogue or, where the linear does not take it, gate and up [rows, N]
+    // from the two halves of the weight.
     const size_t es = in->elementSize(), xb = (rows * K * es + 255) / 256 * 256;
-    const size_t gb = swiglu ? (rows * N * es + 255) / 256 * 256 : 0;
-    char *ws = static_cast<char *>(device::amd::workspace(
-                   in->deviceId(), kernels::kScratchReserved + xb + 2 * gb)) +
-               kernels::kScratchReserved;
+    kernels::LinearCall call{out->data(), nullptr, weight->data(), sc, bp, rows, K, N, swiglu, in->dtype()};
+    const bool halves = swiglu && !kernels::linearSwigluFused(call);
+    const size_t gb = halves ? (rows * N * es + 255) / 256 * 256 : 0, head = xb + 2 * gb;
+    call.swiglu = swiglu && !halves;
+    size_t spare = 0;
+    char *ws = linearScratch(in->deviceId(), head, kernels::linearWorkspaceBytes(call), spare, s);
     kernels::rmsNorm(ws, ro, in->data(), ri, norm_weight->data(), rows, K, eps, in->dtype(), s);
-    if (!swiglu) {
-        kernels::linear(out->data(), ws, weight->data(), sc, bp, rows, K, N, in->dtype(), s);
+    call.x = ws;
+    if (!halves) {
+        kernels::linear(call, ws + head, spare, s);
     } else {
-        const size_t wb = N * K * weight->elementSize();
         char *g = ws + xb, *u = ws + xb + gb;
-        kernels::linear(g, ws, weight->data(), sc, bp, rows, K, N, in->dtype(), s);
-        kernels::linear(u, ws, weight->data() + wb, sc ? sc + N : nullptr,
-                        bp ? static_cast<const char *>(bp) + N * es : nullptr, rows, K, N,
-                        in->dtype(), s);
+        call.out = g;
+        kernels::linear(call, ws + head, spare, s);
+        call.out = u;
+        call.w = weight->data() + N * K * weight->elementSize();
+        if (sc) call.scale = sc + N;
+        if (bp) call.bias = static_cast<const char *>(bp) + N * es;
+        kernels::linear(call, ws + head, spare, s);
         kernels::swiglu(out->data(), g, u, rows * N, in->dtype(), s);
     }
     launched("rmsNormLinear (composed)");
