@@ -17,13 +17,7 @@
 //  - M <= 16, linearSkinny: HBM-bound; a block owns 16 channels, its waves split K, load
 //    weight rows row-contiguously and transpose them through a per-wave LDS tile into
 //    v_mfma_f32_16x16x32 operands; partials summed in LDS in wave order.
-//  - more rows (prefill): MFMA-bound, v_mfma_f32_32x32x16 on 128 x 128 output tiles of 8
-//    waves computing out^T = w x^T (each lane ends with 4 consecutive channels of one row).
-//    linearDirect (16-bit weights, K % 64 == 0) moves the operands HBM -> LDS with
-//    global_load_lds_dwordx4 through 3 stages and XOR-swizzled rows; linearTiled (INT8
-//    weights or other K) stages them through registers and a padded LDS tile, converting
-//    INT8 codes to exact bf16 / f16 on the way.  Blocks map to the 8 XCDs so that a weight
-//    tile stays in one L2 while the row tiles pass over it.
+//  - more rows (prefill): linear_gemm.hip, MFMA tiles.
 //  - f32: linearGemvRow / linearGemv for one row, linear_gemm.hip for more (K % 4 == 0).
 //  - anything else (unaligned rows, K not a multiple of a 16-byte chunk, f32 against INT8
 //    weights): linearScalar, one thread per output with the reference's sequential sum.
@@ -43,7 +37,6 @@ namespace llaisys::kernels {
 namespace {
 
 using namespace lin;
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 struct LinearArgs {
     void *out;
@@ -53,275 +46,6 @@ struct LinearArgs {
     const void *bias;    // T, or null
     int M, N, K;
 };
-
-// 32 x 32 x 16: A[m = l % 32][k = 8 (l / 32) + j], B[k = 8 (l / 32) + j][n = l % 32],
-// D[m = 8 (i / 4) + 4 (l / 32) + i % 4][n = l % 32]; twice the sustained rate of 16 x 16 x 32
-template <typename T>
-__device__ __forceinline__ f32x16 mfma32(const v4u &a, const v4u &b, const f32x16 &c) {
-    if constexpr (std::is_same_v<T, BF16>)
-        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-    else
-        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-}
-
-// Many rows (prefill): MFMA-bound.  A block of NWW x NWX waves owns BW output channels x BX rows;
-// per stage of 64 k it stages both tiles in LDS (row-contiguous global loads, 144-byte row
-// pitch: the MFMA-operand reads and the tile writes are bank-conflict-free), double-buffered
-// with the next stage's global loads in flight during the MFMAs.  The MFMA computes
-// out^T = w x^T: weight rows are the A operand and activation rows the B operand, so each
-// lane ends with 4 consecutive output channels of one row (one 8-byte store).  INT8 codes
-// are converted to exact bf16 / f16 values on their way into LDS.
-constexpr int kTK = 64;               // k per stage
-constexpr int kXcds = 8;              // accelerator complex dies of an MI355X
-
-// Workgroup barrier for LDS hand-offs only: waits for this wave's LDS accesses, not for its
-// global loads (__syncthreads' fence would also drain the prefetches in flight).  The
-// memory clobber keeps the compiler from moving accesses across it.
-constexpr int kTPitch = 2 * kTK + 16; // LDS row pitch (bytes)
-
-// Epilogue of the tiled kernels: D[8 q + 4 h + e][r32] of 32 x 32 tile (i, j) (q, e < 4) is
-// out[row xr + 32 j + r32][channel wr + 32 i + 8 q + 4 h + e], 4 consecutive channels per
-// (q, lane): scale (INT8), bias, one 8-byte store (or element stores at the edge).
-template <typename T, bool kInt8, int TW, int TX>
-__device__ __forceinline__ void storeTiles(const LinearArgs &a, const f32x16 (&acc)[TW][TX], int wr, int xr, int lane) {
-    const int r32 = lane % 32, h2 = lane / 32;
-    const bool vec = a.N % 4 == 0;
-    using C = std::conditional_t<std::is_same_v<T, BF16>, Bf16Cvt, F16Cvt>;
-#pragma unroll
-    for (int i = 0; i < TW; ++i)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int n = wr + 32 * i + 8 * q + 4 * h2;
-            float sc[4], bv[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int ne = min(n + e, a.N - 1);
-                sc[e] = kInt8 ? a.scale[ne] : 1.0f;
-                bv[e] = a.bias ? Fmt<T>::get(a.bias, ne) : 0.0f;
-            }
-#pragma unroll
-            for (int j = 0; j < TX; ++j) {
-                const int m = xr + 32 * j + r32;
-                if (m >= a.M) continue;
-                float v[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float sum = kInt8 ? sc[e] * acc[i][j][4 * q + e] : acc[i][j][4 * q + e];
-                    v[e] = a.bias ? sum + bv[e] : sum;
-                }
-                if (vec && n + 3 < a.N) {
-                    const uint32_t lo = C::narrow(v[0]) | (C::narrow(v[1]) << 16);
-                    const uint32_t hi = C::narrow(v[2]) | (C::narrow(v[3]) << 16);
-                    *reinterpret_cast<v2u *>(static_cast<char *>(a.out) + (size_t(m) * a.N + n) * 2) = v2u{lo, hi};
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (n + e < a.N) Fmt<T>::put(a.out, size_t(m) * a.N + n + e, v[e]);
-                }
-            }
-        }
-}
-
-template <typename T, bool kInt8, int BW, int BX, int NWW, int NWX, int P>
-__global__ void __launch_bounds__(NWW * NWX * 64)
-    linearTiled(LinearArgs a) {
-    constexpr int NT = NWW * NWX * kWave;         // threads
-    constexpr int WW = BW / NWW, WX = BX / NWX;   // wave tile (NWW x NWX waves)
-    constexpr int TW = WW / 32, TX = WX / 32;     // 32 x 32 MFMA tiles per wave
-    constexpr int kXRows = NT / 8;                // 16-bit rows: 8 lanes x 16 B
-    constexpr int kXLoads = BX / kXRows;
-    constexpr int kWRows = kInt8 ? NT / 4 : NT / 8; // INT8 rows: 4 lanes x 16 codes
-    constexpr int kWLoads = BW / kWRows;
-    static_assert(kXLoads >= 1 && kWLoads >= 1 && TW >= 1 && TX >= 1, "tile too small for the block");
-    static_assert(BX % kXRows == 0 && BW % kWRows == 0, "the load passes must cover the tile rows");
-    __shared__ __align__(16) char lds[2][(BW + BX) * kTPitch];
-    const int tid = int(threadIdx.x);
-    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
-    const int lane = tid % kWave;
-    // Blocks are dispatched to the 8 XCDs round-robin, each XCD with its own L2: give each
-    // XCD a contiguous range of weight tiles and walk the activation tiles fastest inside it,
-    // so that a weight tile stays in that L2 while every row tile passes over it.
-    const int nbx = (a.M + BX - 1) / BX;
-    const int nb = int(gridDim.x), b = int(blockIdx.x);
-    const int v = nb % kXcds == 0 ? (b % kXcds) * (nb / kXcds) + b / kXcds : b;
-    const int bx = v % nbx, bw = v / nbx;
-    const int w0 = bw * BW, x0 = bx * BX;
-    const int ww0 = (wave % NWW) * WW, wx0 = (wave / NWW) * WX;
-    const char *xb = static_cast<const char *>(a.x);
-    const char *wb = static_cast<const char *>(a.w);
-    const int nk = (a.K + kTK - 1) / kTK;
-
-    // global loads of stage kt: activation rows (t / 8 + 32 i, chunk t % 8) and weight rows
-    const int xr = tid / 8, xc = tid % 8;
-    const int wr = tid / (NT / kWRows), wc = tid % (NT / kWRows);
-    // global loads of stage kt into ring slot r; past the last stage: the last stage again
-    // (loads stay unconditional, so that the compiler keeps them where they are issued)
-    v4u gx[P][kXLoads], gw[P][kWLoads];
-    const auto loadGlobal = [&](int kt, v4u(&rx)[kXLoads], v4u(&rw)[kWLoads]) {
-        kt = min(kt, nk - 1);
-        const int kx = kt * kTK + 8 * xc;
-        const bool xin = kx < a.K; // K % 8 == 0
-#pragma unroll
-        for (int i = 0; i < kXLoads; ++i) {
-            const int row = min(x0 + xr + kXRows * i, a.M - 1);
-            rx[i] = *reinterpret_cast<const v4u *>(xb + (size_t(row) * a.K + (xin ? kx : 0)) * 2);
-            if (!xin) rx[i] = v4u{0u, 0u, 0u, 0u};
-        }
-        const int kw = kt * kTK + (kInt8 ? 16 : 8) * wc;
-        const bool win = kw < a.K; // K % 8 == 0 (16-bit) / K % 16 == 0 (INT8)
-#pragma unroll
-        for (int i = 0; i < kWLoads; ++i) {
-            const int row = min(w0 + wr + kWRows * i, a.N - 1);
-            rw[i] = *reinterpret_cast<const v4u *>(wb + (size_t(row) * a.K + (win ? kw : 0)) * (kInt8 ? 1 : 2));
-            if (!win) rw[i] = v4u{0u, 0u, 0u, 0u};
-        }
-    };
-    const auto storeLds = [&](int buf, const v4u(&rx)[kXLoads], const v4u(&rw)[kWLoads]) {
-        char *base = lds[buf];
-#pragma unroll
-        for (int i = 0; i < kXLoads; ++i)
-            *reinterpret_cast<v4u *>(base + (BW + xr + kXRows * i) * kTPitch + 16 * xc) = rx[i];
-#pragma unroll
-        for (int i = 0; i < kWLoads; ++i) {
-            char *dst = base + (wr + kWRows * i) * kTPitch;
-            if constexpr (kInt8) {
-                *reinterpret_cast<v4u *>(dst + 32 * wc) = codesToT<T>(v2u{rw[i].x, rw[i].y});
-                *reinterpret_cast<v4u *>(dst + 32 * wc + 16) = codesToT<T>(v2u{rw[i].z, rw[i].w});
-            } else {
-                *reinterpret_cast<v4u *>(dst + 16 * wc) = rw[i];
-            }
-        }
-    };
-
-    f32x16 acc[TW][TX];
-#pragma unroll
-    for (int i = 0; i < TW; ++i)
-#pragma unroll
-        for (int j = 0; j < TX; ++j)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
-    const int r32 = lane % 32, h2 = lane / 32;
-
-    // stage 0 to LDS, stages 1..P in flight
-    loadGlobal(0, gx[0], gw[0]);
-    storeLds(0, gx[0], gw[0]);
-#pragma unroll
-    for (int r = 0; r < P; ++r) loadGlobal(1 + r, gx[r], gw[r]);
-    ldsBarrier();
-    for (int base = 0; base < nk; base += P) {
-#pragma unroll
-        for (int r = 0; r < P; ++r) {
-            const int kt = base + r; // stage in LDS; ring slot r holds stage kt + 1
-            if (kt >= nk) break;
-            const char *tile = lds[kt & 1];
-#pragma unroll
-            for (int st = 0; st < kTK / 16; ++st) {
-                v4u fa[TW], fb[TX];
-#pragma unroll
-                for (int i = 0; i < TW; ++i)
-                    fa[i] = *reinterpret_cast<const v4u *>(tile + (ww0 + 32 * i + r32) * kTPitch + 32 * st + 16 * h2);
-#pragma unroll
-                for (int j = 0; j < TX; ++j)
-                    fb[j] = *reinterpret_cast<const v4u *>(tile + (BW + wx0 + 32 * j + r32) * kTPitch + 32 * st + 16 * h2);
-#pragma unroll
-                for (int i = 0; i < TW; ++i)
-#pragma unroll
-                    for (int j = 0; j < TX; ++j) acc[i][j] = mfma32<T>(fa[i], fb[j], acc[i][j]);
-            }
-            // stage kt + 1 (past the end: harmless, nothing reads it) into the other buffer,
-            // whose last readers finished before the previous barrier; then refill the slot
-            storeLds((kt + 1) & 1, gx[r], gw[r]);
-            loadGlobal(kt + 1 + P, gx[r], gw[r]);
-            ldsBarrier();
-        }
-    }
-
-    storeTiles<T, kInt8, TW, TX>(a, acc, w0 + ww0, x0 + wx0, lane);
-}
-
-// Many rows, 16-bit weights, K a multiple of 64: the tiled kernel's MFMA work with the
-// operands moved HBM -> LDS by global_load_lds_dwordx4 (no register staging, no LDS write
-// instructions) through S stages (S - 1 in flight while the MFMAs run on one).  A load
-// instruction fills 1 KB of LDS contiguously (8 rows x 128 B, one 64-k stage of a row),
-// so rows cannot be padded; instead the lane that fills slot c of row r fetches k-chunk
-// c ^ ((r >> 1) & 7), and the MFMA-operand reads apply the same XOR (bank-conflict-free,
-// measured).  Waits count this wave's loads (vmcnt) and one LDS-only barrier per stage
-// makes every wave's loads visible and frees the stage read two steps ago.
-template <typename T, int BW, int BX, int NWW, int NWX, int S>
-__global__ void __launch_bounds__(NWW * NWX * 64)
-    linearDirect(LinearArgs a) {
-    constexpr int NWV = NWW * NWX;
-    constexpr int WW = BW / NWW, WX = BX / NWX, TW = WW / 32, TX = WX / 32;
-    constexpr int kRowB = 2 * kTK;                 // bytes of a row per stage
-    constexpr int kStageB = (BW + BX) * kRowB;
-    constexpr int kLoads = (BW + BX) / 8 / NWV;    // loads (8 rows each) per wave per stage
-    static_assert((BW + BX) % (8 * NWV) == 0 && kLoads * (S - 2) < 64, "load split");
-    __shared__ __align__(16) char lds[S * kStageB];
-    const int tid = int(threadIdx.x), lane = tid % kWave;
-    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
-    const int nbx = (a.M + BX - 1) / BX;
-    const int nb = int(gridDim.x), b = int(blockIdx.x);
-    const int v = nb % kXcds == 0 ? (b % kXcds) * (nb / kXcds) + b / kXcds : b;
-    const int bx = v % nbx, bw = v / nbx;
-    const int w0 = bw * BW, x0 = bx * BX;
-    const int ww0 = (wave % NWW) * WW, wx0 = (wave / NWW) * WX;
-    const char *xb = static_cast<const char *>(a.x), *wb = static_cast<const char *>(a.w);
-    const int nk = a.K / kTK;
-    // tile rows [0, BW) are weight rows, [BW, BW + BX) activation rows (clamped at the edges)
-    const char *src[kLoads];
-#pragma unroll
-    for (int i = 0; i < kLoads; ++i) {
-        const int tr = 8 * (wave * kLoads + i) + lane / 8;
-        const int kc = (lane % 8) ^ ((tr >> 1) & 7);
-        src[i] = tr < BW ? wb + (size_t(min(w0 + tr, a.N - 1)) * a.K + 8 * kc) * 2
-                         : xb + (size_t(min(x0 + tr - BW, a.M - 1)) * a.K + 8 * kc) * 2;
-    }
-    const auto issue = [&](int kt) { // past the last stage: the last stage again, never read
-        const int ktc = min(kt, nk - 1);
-        char *dst = lds + (kt % S) * kStageB;
-#pragma unroll
-        for (int i = 0; i < kLoads; ++i)
-            __builtin_amdgcn_global_load_lds(
-                (const void __attribute__((address_space(1))) *)(src[i] + size_t(ktc) * kRowB),
-                (void __attribute__((address_space(3))) *)(dst + 8 * (wave * kLoads + i) * kRowB), 16, 0, 0);
-    };
-    f32x16 acc[TW][TX];
-#pragma unroll
-    for (int i = 0; i < TW; ++i)
-#pragma unroll
-        for (int j = 0; j < TX; ++j)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
-    const int r32 = lane % 32, h2 = lane / 32;
-#pragma unroll
-    for (int st = 0; st < S - 1; ++st) issue(st);
-    for (int kt = 0; kt < nk; ++kt) {
-        waitVmcnt<kLoads * (S - 2)>(); // this wave's loads of stage kt have landed
-        ldsBarrier();                  // every wave's have; stage kt - 1 is no longer read
-        issue(kt + S - 1);
-        const char *tile = lds + (kt % S) * kStageB;
-#pragma unroll
-        for (int st = 0; st < kTK / 16; ++st) {
-            v4u fa[TW], fb[TX];
-#pragma unroll
-            for (int i = 0; i < TW; ++i) {
-                const int row = ww0 + 32 * i + r32;
-                fa[i] = *reinterpret_cast<const v4u *>(tile + row * kRowB + 16 * ((2 * st + h2) ^ ((row >> 1) & 7)));
-            }
-#pragma unroll
-            for (int j = 0; j < TX; ++j) {
-                const int row = BW + wx0 + 32 * j + r32;
-                fb[j] = *reinterpret_cast<const v4u *>(tile + row * kRowB + 16 * ((2 * st + h2) ^ ((row >> 1) & 7)));
-            }
-#pragma unroll
-            for (int i = 0; i < TW; ++i)
-#pragma unroll
-                for (int j = 0; j < TX; ++j) acc[i][j] = mfma32<T>(fa[i], fb[j], acc[i][j]);
-        }
-    }
-    waitVmcnt<0>(); // no LDS write may still be landing when the wave ends
-    storeTiles<T, false, TW, TX>(a, acc, w0 + ww0, x0 + wx0, lane);
-}
 
 // Few rows (M <= 16, decode): HBM-bound on the weights; the skinny MFMA loop of
 // linear_common.hpp over one set of 16 channels, x rows >= M entering as zeros.  The waves'
@@ -598,29 +322,6 @@ void launch(const LinearArgs &a, hipStream_t s) {
                 const size_t lds = size_t(nw) * (16 * skinnyPitch(kInt8) + 256 * sizeof(float));
                 linearSkinny<T, kInt8><<<unsigned(tiles), unsigned(nw * kWave), lds, s>>>(a);
                 return;
-            }
-            // tile shape: 128 x 128 (8 waves, 2 stages of loads in flight) while that still
-            // gives most CUs a block, else 64 x 64
-            const auto blocks = [&](int bw, int bx) {
-                return unsigned((a.N + bw - 1) / bw) * unsigned((a.M + bx - 1) / bx);
-            };
-            if (blocks(128, 128) >= 192) {
-                // 16-bit weights: 96 x 128 tiles (4 waves of 96 x 32, 4 stages) when 128 x 128
-                // tiles leave CUs idle in a single round and the narrower tiles still fit one:
-                // prefill 2048 x 8960 -> 1536 (192 vs 256 tiles) 73.9 -> 69.9 us, the same bits
-                // Grids of 512+ tiles: 4 waves of 64 x 64 and 2 stages (64 KB of LDS, two blocks
-                // per CU): prefill 2048 x 1536 -> 8960 85.2 -> 73.7 us, 4096 rows 166 -> 143 us
-                // (with one or two blocks per CU the 3-stage 8-wave form stays ahead)
-                if (!kInt8 && a.K % kTK == 0 && blocks(128, 128) < 256 && blocks(96, 128) <= 256)
-                    linearDirect<T, 96, 128, 1, 4, 4><<<blocks(96, 128), 256, 0, s>>>(a);
-                else if (!kInt8 && a.K % kTK == 0 && blocks(128, 128) >= 512)
-                    linearDirect<T, 128, 128, 2, 2, 2><<<blocks(128, 128), 256, 0, s>>>(a);
-                else if (!kInt8 && a.K % kTK == 0)
-                    linearDirect<T, 128, 128, 4, 2, 3><<<blocks(128, 128), 512, 0, s>>>(a);
-                else
-                    linearTiled<T, kInt8, 128, 128, 4, 2, 2><<<blocks(128, 128), 512, 0, s>>>(a);
-            } else {
-                linearTiled<T, kInt8, 64, 64, 2, 2, 2><<<blocks(64, 64), 256, 0, s>>>(a);
             }
         }
         return;

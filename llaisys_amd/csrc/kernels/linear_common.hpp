@@ -35,7 +35,7 @@ __device__ __forceinline__ v4u codesToT(const v2u &c) {
         const int sh = 16 * (e % 2);
         const float lo = float(int8_t(src >> sh)), hi = float(int8_t(src >> (sh + 8)));
         if constexpr (std::is_same_v<T, BF16>)
-            w[e] = (__float_as_uint(lo) >> 16) | (__float_as_uint(hi) & 0xFFFF0000u); // exact: 8-bit values
+            w[e] = __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u); // exact: 8-bit values
         else
             w[e] = f32ToF16(lo) | (f32ToF16(hi) << 16);
     }

@@ -1,0 +1,8 @@
+// Tiled linear layers in bf16: instantiations of linear_gemm_kernels.hpp.
+#include "linear_gemm_kernels.hpp"
+
+namespace llaisys::kernels {
+
+void gemmBf16(GemmTile t, const GemmArgs &a, bool swiglu, hipStream_t s) { gemm16<BF16>(t, a, swiglu, s); }
+
+} // namespace llaisys::kernels

@@ -8,8 +8,10 @@ import pytest
 
 import llaisys_amd as L
 import oracle
+from llaisys_amd.hostfmt import f32_to_bf16
 from numerics import assert_exact, assert_linear_close
-from test_linear_gpu import AMD, DTS, dev, linear, sample
+from test_norm_linear_gpu import Case
+from test_linear_gpu import AMD, DTS, dev, int8_weights, linear, linear_w8a16, sample
 
 pytestmark = pytest.mark.gpu
 
@@ -27,6 +29,50 @@ def test_f32_tiles(shape):
     got = linear(x, w, b, "f32")
     assert_linear_close(got, oracle.linear(x, w, b), x, w, f"f32 {shape}")
     assert_exact(linear(x, w, b, "f32"), got, "repeat")
+
+
+# rows, in_features, out_features of the 16-bit tiles: the 64-row tile with its deep stages (first and
+# last row count, K of one chunk pair, a ragged last stage, split), then the tiles that the expected
+# launch time picks as the rows grow (64 x 64, 128 x 64, 96 x 128, 128 x 128, 192 x 128, 256 x 128,
+# 192 x 256), each with ragged channels or rows, one stage or a ragged last one, and split
+EDGES = [(17, 16, 64), (64, 144, 63), (37, 1552, 130), (64, 8960, 66), (65, 16, 65), (96, 208, 300), (128, 8960, 192),
+         (161, 1552, 2000), (300, 4112, 140), (300, 64, 9002), (800, 80, 9001), (1024, 2064, 770), (1500, 96, 1531),
+         (2047, 48, 9003), (3999, 112, 1540), (2048, 64, 18000)]
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("shape", EDGES, ids=lambda s: "x".join(map(str, s)))
+def test_16_bit_tiles(shape, dt):
+    """Dense against the oracle, and W8A16 with unit scales over the same codes bit for bit (one
+    order of the sums); W8A16 with scales and bias against the oracle."""
+    rows, in_f, out_f = shape
+    rng = np.random.default_rng(zlib.crc32(repr((shape, dt)).encode()))
+    x, b = sample(rng, (rows, in_f), dt), sample(rng, (out_f,), dt)
+    codes, scale = int8_weights(rng, out_f, in_f)
+    w = f32_to_bf16(codes.astype(np.float32)) if dt == "bf16" else codes.astype(np.float16)
+    some = slice(None) if rows * in_f * out_f < 1 << 30 else np.r_[:70, rows // 2:rows // 2 + 140, rows - 70:rows]
+    xs = x[some]
+    got = linear(x, w, b, dt)
+    assert_linear_close(got[some], oracle.linear(xs, w, b), xs, w, f"{dt} {shape}")
+    assert_exact(linear_w8a16(x, codes, np.ones(out_f, np.float32), b, dt), got, "unit scales")
+    assert_linear_close(linear_w8a16(x, codes, scale, b, dt)[some], oracle.linear_w8a16(xs, codes, scale, b), xs, codes,
+                        f"w8a16 {dt} {shape}", w_scale=scale)
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16", "f32"])
+@pytest.mark.parametrize("rows, in_f, out_f", [(2, 64, 100), (17, 528, 90), (64, 2064, 33), (100, 1536, 131), (300, 528, 1000),
+                                               (1100, 144, 4500)])
+def test_swiglu_epilogue_equals_separate_ops(rows, in_f, out_f, dt):
+    """rms_norm -> gate / up -> swiglu with the swiglu in the linear's epilogue (or in its split
+    reduction) equals the three ops on the two halves of the weight, bit for bit."""
+    for int8 in (False, True):
+        if int8 and (dt == "f32" or in_f % 16):
+            continue
+        c = Case(rows, in_f, out_f, dt, int8, True, bias=True, res=True, seed=rows)
+        got, h = c.fused()
+        want, _, h_want = c.composed()
+        assert_exact(h, h_want, "residual")
+        assert_exact(got, want, f"int8={int8}")
 
 
 def test_split_k_under_capture_without_workspace(monkeypatch):
