@@ -15,17 +15,13 @@
 // tests bound the difference by the f32 accumulation error of the reference itself.
 //
 // Design, three kernels (the launcher at the end picks one):
-//  - attnMfmaLds / attnMfma (bf16, head_dim 128, >= 16 queries: prefill): MFMA-bound; 16
-//    queries x one kv head's q heads per block, S^T = K Q^T and O^T += V^T P^T on
-//    v_mfma_f32_16x16x32_bf16 with K / V tiles in LDS one tile ahead; with few blocks per CU,
-//    two wave sets per block split the key tiles (kSplit).  attnMfmaLds moves bf16 tiles
-//    HBM -> LDS directly; an INT8 cache whose bf16 form fits the workspace is dequantized
-//    once into it and attended by it as bf16 (the same operands), and attnMfma stages other
-//    INT8 caches through registers, converting the codes on the way.
+//  - attnPrefill (bf16 / f16, head_dim 64 or 128, >= 16 queries): 32 queries of two q heads per
+//    block on v_mfma_f32_32x32x16, the keys split over the block's waves and, where the blocks
+//    leave CUs idle, over blocks (merged by attnCombineFew / attnCombine).
 //  - attnDecodeMfma (bf16 q, head_dim 128, fewer queries: decode, cache in bf16 or INT8):
 //    HBM-bound; the key range is cut into chunks, one block per (query, kv head, chunk) with
 //    the kv head's q heads as the MFMA columns; attnCombine merges the chunk partials.
-//  - attnGroup (other dtypes, head_dim 64): one wavefront per q head, the waves of a block
+//  - attnGroup (f32, fewer queries in f16 or with head_dim 64): one wavefront per q head, the waves of a block
 //    being q heads of one kv head (they read the same K / V rows).  A key row of D elements
 //    is spread over R = D / 8 lanes, 8 elements per lane, so one load instruction covers
 //    64 / R keys; per batch of U instructions the wave forms its scores (8 FMAs, a butterfly
@@ -427,500 +423,340 @@ __device__ __forceinline__ v4u codesToBf16(const v4u &raw, float sc) {
                Bf16Cvt::narrow2Q(cv(uy, 0), cv(uy, 1)), Bf16Cvt::narrow2Q(cv(uy, 2), cv(uy, 3))};
 }
 
-// ---- prefill on MFMA (bf16 q / out, head_dim 128, cache in bf16 or INT8) --------------
-// One block per (16 queries, kv head, slice of W q heads), one wave per q head.  Per tile
-// of 64 keys a wave forms S^T = K Q^T with v_mfma_f32_16x16x32_bf16 (A = 16 key rows of
-// the tile, B = the wave's 16 queries kept in registers), so each lane holds the scores of
-// one query (column l % 16) for 16 of the keys and the softmax needs only an exchange
-// between the 4 lanes of that column; then O^T += V^T P^T with the same instruction.
-// Operand layouts (measured on MI355X): A[m = l % 16][k = 8(l / 16) + j],
-// B[k = 8(l / 16) + j][n = l % 16], D[m = 4(l / 16) + i][n = l % 16].
-// Key order: row m of score tile t (of 4) is key 32(t / 2) + 8(m / 4) + 4(t % 2) + m % 4,
-// so lane group g holds keys 32p + 8g .. + 7 of tiles 2p and 2p + 1 -- exactly the 8
-// consecutive k-slots 8g + j of the P V product for keys 32p .. 32p + 31, and the V^T
-// operand of those slots is one 16-byte LDS read.  P enters as bf16 hi + lo parts (2^-17
-// relative), so the output keeps f32 accuracy.
+// ---- prefill on MFMA (bf16 / f16, head_dim 64 or 128, cache in the type or INT8) --------------
+// A block takes 32 queries of 2 q heads of one kv head (odd groups: 64 queries of one q head), a
+// "unit" each, and its 2 x kSplits waves walk the keys in steps of kSplits x 32: wave (unit u,
+// split s) takes keys 32 s .. + 31 of every step, so the splits of a unit stay balanced up to the
+// causal diagonal and merge through LDS at the end.  Per step a wave forms S^T = K Q^T (32 keys x
+// 32 queries) and O^T += V^T P^T with v_mfma_f32_32x32x16: A[m = l % 32][k = 8 (l / 32) + j],
+// B[k = 8 (l / 32) + j][n = l % 32], D[m = 8 (i / 4) + 4 (l / 32) + i % 4][n = l % 32].  Row m =
+// 16 g + 8 a + 4 h + b of K is key 16 g + 8 h + 4 a + b, so lane half h ends with the scores of keys
+// 16 g + 8 h + 0 .. 7 of its query -- the 8 consecutive k of the P V product's B operand -- and the
+// softmax needs one exchange between the two lanes of a query.  P enters as two 16-bit parts (hi +
+// lo: 2^-17 relative in bf16, 2^-22 in f16), so the output keeps f32 accuracy; in f16 the weights
+// carry a factor 2^8, which keeps the parts of small weights normal numbers and cancels in O / l.
+//
+// K and V tiles move HBM -> LDS with global_load_lds_dwordx4 (1 KB per instruction, two stages, the
+// next step's loads in flight during this one's math).  V stays row-major; its transposed operand
+// is two ds_read_b64_tr_b16: within 16 lanes, lane j's element e is element j % 4 of the 8 bytes
+// that lane 4 e + j / 4 addresses.  Rows cannot be padded (the load fills LDS contiguously), so the
+// 16-byte chunks of a row are XOR-swizzled: K so that 16 rows' reads of one chunk touch all banks,
+// V so that the 64-byte pieces of 4 rows do.  An INT8 cache is dequantized into the workspace when
+// it fits, else its codes are converted on their way into LDS (the same operands, the same bits).
+// Keys past the cache read row 0 (finite wherever the reference's own output is; they weigh 0).
+//
+// What bounds it: a step is 24 MFMAs (768 cycles) and as much VALU work (16 exponentials per lane
+// and their two parts) per wave, two waves on a SIMD walking the same phases between barriers.
+// 2048 queries, 12 / 2 heads, bf16: 44.9 us with 16-query tiles and one wave per q head on 16 x 16
+// x 32 MFMAs (1 KB of LDS read per 16 MFMA cycles, CUs with early queries idle) -> 38.0 us; f16, 300
+// queries over 1500 INT8 keys: 479 us on the vector kernel -> 25.2 us.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef uint32_t v2u __attribute__((ext_vector_type(2)));
+typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 
-constexpr int kMfmaQ = 16;  // queries per block
-constexpr int kMfmaKT = 64; // keys per tile
-constexpr int kKtLd = 136;  // K tile row stride (bf16): 16-byte rows, rows 4 banks apart
-constexpr int kVtLd = 72;   // V^T row stride (bf16): 16-byte reads; rows 8 apart 32 banks apart
+constexpr int kMfmaQ = 16;   // fewest queries that take the prefill kernel
+constexpr int kSplits = 4;   // waves per unit, each with 32 keys of a step
+constexpr int kStepKeys = 32 * kSplits;
 
 __device__ __forceinline__ bf16x8 asBf16x8(const v4u &r) { return __builtin_bit_cast(bf16x8, r); }
 
-// Tiles move HBM -> registers -> LDS with one tile of lookahead: while the waves compute on
-// tile t (in LDS buffer t % 2), every thread holds its share of tile t + 1 in registers and
-// writes it to the other buffer at the start of the next step, so the loads overlap the
-// MFMA work and a step needs one barrier.  K is stored as loaded (row-major); V is stored
-// transposed from pairs of consecutive keys, one 4-byte write per column and pair (the 32
-// lanes of a pair of rows write 32 consecutive words, the other 32 lanes rows 32 banks on).
-// kSplit: the block holds two waves per q head, and the key tiles are cut in two halves that
-// the two wave sets walk in lockstep (one barrier per step for both), each staging its own
-// tiles; at the end the second half's (max, sum, output) is merged into the first's through
-// LDS.  It halves the longest block's chain of tiles -- the causal imbalance that bounds
-// a prefill with about one block per CU.
-template <int W, bool kSplit, bool kInt8>
-__global__ void __launch_bounds__(kWave * W * (kSplit ? 2 : 1))
-    attnMfma(AttnArgs a) {
-    constexpr int D = 128, KB = D / 32, DT = D / 16;
-    constexpr int NHALF = kSplit ? 2 : 1;
-    constexpr int kKItems = kMfmaKT * (D / 8);           // 16-byte K pieces per tile
-    constexpr int kVItems = (kMfmaKT / 2) * (D / 8);     // V pieces: 2 keys x 8 columns
-    constexpr int kKPer = (kKItems + kWave * W - 1) / (kWave * W);
-    constexpr int kVPer = (kVItems + kWave * W - 1) / (kWave * W);
-    __shared__ uint16_t kt_all[NHALF][2][kMfmaKT][kKtLd];
-    __shared__ uint16_t vt_all[NHALF][2][D][kVtLd];
-    const int wave_all = __builtin_amdgcn_readfirstlane(int(threadIdx.x) / kWave);
-    const int half = kSplit ? wave_all / W : 0;   // key half this wave walks
-    const int wave = wave_all % W;                 // q head of the slice
-    const int ltid = int(threadIdx.x) % (kWave * W); // thread index within the half
-    auto &kt = kt_all[half];
-    auto &vt = vt_all[half];
-    const int lane = int(threadIdx.x) % kWave;
-    const int n = lane % 16, g4 = lane / 16;
-
-    const size_t nqb = (a.seq + kMfmaQ - 1) / kMfmaQ;
-    unsigned b = blockIdx.x;
-    const int sl = int(b % unsigned(a.slices));
-    b /= unsigned(a.slices);
-    const int g = int(b % unsigned(a.nkvh));
-    const size_t qb = nqb - 1 - size_t(b / unsigned(a.nkvh)); // latest queries first
-    const int h = g * a.group + sl * W + wave;
-    const size_t q0 = qb * kMfmaQ;
-    const size_t qi = min(q0 + size_t(n), a.seq - 1); // this lane's query (clamped for loads)
-    const size_t vis_q = visibleKeys(a.total, a.seq, qi);
-    const size_t vis_blk = visibleKeys(a.total, a.seq, min(q0 + kMfmaQ - 1, a.seq - 1));
-    const size_t vis_first = visibleKeys(a.total, a.seq, q0); // the fewest keys any query sees
-    const size_t ntiles = (vis_blk + kMfmaKT - 1) / kMfmaKT;
-    const float c2 = a.scale * 1.4426950408889634f; // scores to base-2 exponents
-
-    bf16x8 qreg[KB];
-#pragma unroll
-    for (int kb = 0; kb < KB; ++kb) {
-        const uint16_t *qp = static_cast<const uint16_t *>(a.q) + (qi * a.nh + h) * D + 32 * kb + 8 * g4;
-        qreg[kb] = asBf16x8(*reinterpret_cast<const v4u *>(qp));
-    }
-    float m = -INFINITY, lsum = 0.0f; // m: running max of the raw dots (scaled by c2 in use)
-    f32x4 o[DT];
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) o[dt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-
-    // cache rows of the kv head: row t at element (t * nkvh + g) * D; INT8 codes with one
-    // scale per (t, g), turned into bf16(code * scale) (codesToBf16) when staged into LDS
-    const size_t rstride = size_t(a.nkvh);
-    v4u kraw[kKPer], vraw[kVPer][2];
-    float ksc[kInt8 ? kKPer : 1], vsc[kInt8 ? kVPer : 1][2];
-    const auto loadTile = [&](size_t t0) {
-        const size_t left = a.total - t0; // keys of the cache from t0 on (> 0)
-#pragma unroll
-        for (int r = 0; r < kKPer; ++r) {
-            const int idx = ltid + r * kWave * W;
-            const int kk = idx / (D / 8), col = 8 * (idx % (D / 8));
-            kraw[r] = v4u{0u, 0u, 0u, 0u}; // keys past the cache: zeros
-            if constexpr (kInt8) ksc[r] = 0.0f;
-            if (idx < kKItems && size_t(kk) < left) {
-                kraw[r] = loadRow8<kInt8>(a.k, (t0 + kk) * rstride + g, col);
-                if constexpr (kInt8) ksc[r] = a.ks[(t0 + kk) * rstride + g];
-            }
-        }
-#pragma unroll
-        for (int r = 0; r < kVPer; ++r) {
-            const int idx = ltid + r * kWave * W;
-            const int kp = idx % (kMfmaKT / 2), col = 8 * (idx / (kMfmaKT / 2));
-#pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                vraw[r][e] = v4u{0u, 0u, 0u, 0u};
-                if constexpr (kInt8) vsc[r][e] = 0.0f;
-                if (idx < kVItems && size_t(2 * kp + e) < left) {
-                    vraw[r][e] = loadRow8<kInt8>(a.v, (t0 + 2 * kp + e) * rstride + g, col);
-                    if constexpr (kInt8) vsc[r][e] = a.vs[(t0 + 2 * kp + e) * rstride + g];
-                }
-            }
-        }
-    };
-    const auto storeTile = [&](int buf) {
-        if constexpr (kInt8) {
-#pragma unroll
-            for (int r = 0; r < kKPer; ++r) kraw[r] = codesToBf16(kraw[r], ksc[r]);
-#pragma unroll
-            for (int r = 0; r < kVPer; ++r)
-#pragma unroll
-                for (int e = 0; e < 2; ++e) vraw[r][e] = codesToBf16(vraw[r][e], vsc[r][e]);
-        }
-#pragma unroll
-        for (int r = 0; r < kKPer; ++r) {
-            const int idx = ltid + r * kWave * W;
-            if (idx < kKItems)
-                *reinterpret_cast<v4u *>(&kt[buf][idx / (D / 8)][8 * (idx % (D / 8))]) = kraw[r];
-        }
-#pragma unroll
-        for (int r = 0; r < kVPer; ++r) {
-            const int idx = ltid + r * kWave * W;
-            if (idx >= kVItems) continue;
-            const int kp = idx % (kMfmaKT / 2), col = 8 * (idx / (kMfmaKT / 2));
-            const uint32_t w0[4] = {vraw[r][0].x, vraw[r][0].y, vraw[r][0].z, vraw[r][0].w};
-            const uint32_t w1[4] = {vraw[r][1].x, vraw[r][1].y, vraw[r][1].z, vraw[r][1].w};
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                // columns col + 2e (low halves) and col + 2e + 1 (high halves) of keys 2kp, 2kp + 1
-                *reinterpret_cast<uint32_t *>(&vt[buf][col + 2 * e][2 * kp]) =
-                    __builtin_amdgcn_perm(w1[e], w0[e], 0x05040100u);
-                *reinterpret_cast<uint32_t *>(&vt[buf][col + 2 * e + 1][2 * kp]) =
-                    __builtin_amdgcn_perm(w1[e], w0[e], 0x07060302u);
-            }
-        }
-    };
-
-    // this half's tiles: [tbeg, tbeg + tcount); both halves step nsteps times
-    const size_t nsteps = kSplit ? (ntiles + 1) / 2 : ntiles;
-    const size_t tbeg = half ? nsteps : 0;
-    const size_t tcount = half ? ntiles - nsteps : nsteps;
-    if (tcount > 0) loadTile(tbeg * kMfmaKT);
-    for (size_t it = 0; it < nsteps; ++it) {
-        const int buf = int(it & 1);
-        const size_t ti = tbeg + it;
-        const size_t kt0 = ti * kMfmaKT;
-        storeTile(buf);
-        if (it + 1 < tcount) loadTile(kt0 + kMfmaKT); // in flight during this step's math
-        __syncthreads(); // tile ti in LDS; every wave is past the step that read buf last
-        if (kSplit && it >= tcount) continue; // the shorter half idles through its last step
-        // keys of this lane's query visible in the tile: offsets < nvis.  A tile every query
-        // of the block sees whole (all but the causal diagonal) skips the masking.
-        const bool whole = kt0 + kMfmaKT <= vis_first; // block-uniform
-        const int nvis = int(min(vis_q - min(vis_q, kt0), size_t(kMfmaKT)));
-        float p[4][4];
-        float mx = m;
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            const int krow = 32 * (t / 2) + 8 * (n / 4) + 4 * (t % 2) + n % 4; // A row n
-            f32x4 acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int kb = 0; kb < KB; ++kb) {
-                const v4u kv = *reinterpret_cast<const v4u *>(&kt[buf][krow][32 * kb + 8 * g4]);
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(asBf16x8(kv), qreg[kb], acc, 0, 0, 0);
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i) p[t][i] = acc[i];
-        }
-        if (!whole) { // the causal diagonal: keys past this lane's query are masked
-#pragma unroll
-            for (int t = 0; t < 4; ++t)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int off = 32 * (t / 2) + 8 * g4 + 4 * (t % 2) + i; // key of D row 4g + i
-                    p[t][i] = off < nvis ? p[t][i] : -INFINITY;
-                }
-        }
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) mx = fmaxf(mx, p[t][i]);
-        mx = fmaxf(mx, __shfl_xor(mx, 16, kWave));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
-        // exp(scale * (s - max)) as 2^(s * c2 - max * c2); a masked key (-inf) gets weight 0.
-        // Key 0 is visible to every query, so mx = -inf only when every score so far is -inf;
-        // mc = 0 then keeps 2^(-inf - mc) at 0 instead of NaN, with no per-score select.
-        const float mc = mx == -INFINITY ? 0.0f : mx * c2;
-        float ps = 0.0f;
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                p[t][i] = __builtin_amdgcn_exp2f(__builtin_fmaf(p[t][i], c2, -mc));
-                ps += p[t][i];
-            }
-        if (__builtin_expect(__any(mx != m), 0)) { // rescale only when a max moved
-            const float corr = mx == m ? 1.0f : __builtin_amdgcn_exp2f(__builtin_fmaf(m, c2, -mc));
-            lsum *= corr;
-#pragma unroll
-            for (int dt = 0; dt < DT; ++dt) o[dt] *= corr;
-        }
-        m = mx;
-        lsum += ps;
-#pragma unroll
-        for (int p2 = 0; p2 < 2; ++p2) {
-            // P as bf16 hi + lo, two keys per conversion: key 32 p2 + 8g + j is p[2 p2 + j / 4][j % 4]
-            uint32_t hw[4], lw[4];
-#pragma unroll
-            for (int w = 0; w < 4; ++w) {
-                const float x0 = p[2 * p2 + w / 2][2 * (w % 2)], x1 = p[2 * p2 + w / 2][2 * (w % 2) + 1];
-                hw[w] = Bf16Cvt::narrow2Q(x0, x1);
-                lw[w] = Bf16Cvt::narrow2Q(x0 - __uint_as_float(hw[w] << 16), x1 - __uint_as_float(hw[w] & 0xFFFF0000u));
-            }
-            const bf16x8 bhi = asBf16x8(v4u{hw[0], hw[1], hw[2], hw[3]});
-            const bf16x8 blo = asBf16x8(v4u{lw[0], lw[1], lw[2], lw[3]});
-#pragma unroll
-            for (int dt = 0; dt < DT; ++dt) {
-                const v4u vv = *reinterpret_cast<const v4u *>(&vt[buf][16 * dt + n][32 * p2 + 8 * g4]);
-                o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(asBf16x8(vv), bhi, o[dt], 0, 0, 0);
-                o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(asBf16x8(vv), blo, o[dt], 0, 0, 0);
-            }
-        }
-    }
-    float lt = lsum + __shfl_xor(lsum, 16, kWave);
-    lt += __shfl_xor(lt, 32, kWave);
-    if constexpr (kSplit) {
-        // the second half hands (max, sum, output) to its partner wave through LDS (the
-        // tiles' storage, free once every wave is past its last step)
-        float *xch = reinterpret_cast<float *>(&kt_all[0][0][0][0]) + size_t(wave) * kWave * (2 + 4 * DT);
-        __syncthreads();
-        if (half == 1) {
-            xch[lane] = m;
-            xch[kWave + lane] = lt;
-#pragma unroll
-            for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) xch[(2 + 4 * dt + i) * kWave + lane] = o[dt][i];
-        }
-        __syncthreads();
-        if (half == 1) return;
-        const float m1 = xch[lane], l1 = xch[kWave + lane];
-        const float M = fmaxf(m, m1);
-        // a half with no visible key has m = -inf: weight 0 (the other half holds key 0)
-        const float f0 = m == M ? 1.0f : __builtin_amdgcn_exp2f(__builtin_fmaf(m, c2, -M * c2));
-        const float f1 = m1 == M ? 1.0f : __builtin_amdgcn_exp2f(__builtin_fmaf(m1, c2, -M * c2));
-        lt = lt * f0 + l1 * f1;
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) o[dt][i] = o[dt][i] * f0 + xch[(2 + 4 * dt + i) * kWave + lane] * f1;
-    }
-    if (q0 + size_t(n) >= a.seq) return;
-    const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
-    uint16_t *op = static_cast<uint16_t *>(a.out) + (qi * a.nh + h) * D + 4 * g4;
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) {
-        // O^T[d = 16dt + 4g + i][query n]; the reference rounding
-        const uint32_t w0 = f32ToBf16(o[dt][0] * inv) | (f32ToBf16(o[dt][1] * inv) << 16);
-        const uint32_t w1 = f32ToBf16(o[dt][2] * inv) | (f32ToBf16(o[dt][3] * inv) << 16);
-        typedef uint32_t v2u __attribute__((ext_vector_type(2)));
-        *reinterpret_cast<v2u *>(op + 16 * dt) = v2u{w0, w1};
-    }
-}
-
-// ---- prefill on MFMA over a bf16 cache: tiles HBM -> LDS with no register staging -------
-// The arithmetic of attnMfma (same operands, same MFMA order, same bits), with the K and V
-// tiles moved by global_load_lds_dwordx4: one instruction fills 1 KB of LDS (4 key rows of
-// 256 bytes) straight from memory, so a step spends no VALU on staging and holds no tile in
-// registers.  V stays row-major in LDS and the Vᵀ operand of O^T += V^T P^T comes from two
-// ds_read_b64_tr_b16: within each 16 lanes, lane j's element e is element j % 4 of the 8
-// bytes lane 4e + j / 4 addresses (measured on MI355X), so lanes i reading 4 columns
-// 4(i % 4) .. of key row 8g + i / 4 (then + 4) hand lane j of group g the 8 consecutive keys
-// 8g .. 8g + 7 of column j.  Rows cannot be padded (the load fills LDS contiguously), so
-// the 16-byte chunks of each row are XOR-swizzled by row bits: K by (r & 3) | (r >> 3 & 3) << 2,
-// which spreads the 16 rows one ds_read_b128 of an A operand touches over all banks, V by
-// 2 ((r & 3) | (r >> 3 & 1) << 2), which spreads the 8 rows of 32 lanes' transposing reads.
-// Two LDS stages: the loads of tile t + 1 are issued after the barrier that ends every
-// wave's reads of tile t - 1 and land while tile t is computed.  Keys past the cache load
-// row 0 (finite wherever the reference's own output is; masked keys weigh 0).
 typedef short v4s __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ int swzK(int r) { return (r & 3) | (((r >> 3) & 3) << 2); }
 __device__ __forceinline__ int swzV(int r) { return ((r & 3) | (((r >> 3) & 1) << 2)) << 1; }
 __device__ __forceinline__ uint64_t ldsReadTr16(const char *p) {
     const v4s r = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s *)(p));
     return __builtin_bit_cast(uint64_t, r);
 }
 
-template <int W, bool kSplit>
-__global__ void __launch_bounds__(kWave * W * (kSplit ? 2 : 1))
-    attnMfmaLds(AttnArgs a) {
-    constexpr int D = 128, KB = D / 32, DT = D / 16;
-    constexpr int NHALF = kSplit ? 2 : 1;
-    constexpr int kRowB = 2 * D;              // bytes of a key row
-    constexpr int kTileB = kMfmaKT * kRowB;   // one K or V tile
-    constexpr int kLoads = 2 * kTileB / 1024; // 1 KB load instructions per stage
-    constexpr int kPer = (kLoads + W - 1) / W;
-    __shared__ __align__(16) char lds_all[NHALF][2][2 * kTileB]; // [half][stage][K tile | V tile]
-    const int wave_all = __builtin_amdgcn_readfirstlane(int(threadIdx.x) / kWave);
-    const int half = kSplit ? wave_all / W : 0;
-    const int wave = wave_all % W;
-    const int lane = int(threadIdx.x) % kWave;
-    const int n = lane % 16, g4 = lane / 16;
+// Two f32 as two elements of T (hi), and what is left of them as two more (lo)
+template <typename T>
+__device__ __forceinline__ void splitPair(float x0, float x1, uint32_t &hi, uint32_t &lo) {
+    if constexpr (std::is_same_v<T, BF16>) {
+        hi = Bf16Cvt::narrow2Q(x0, x1);
+        lo = Bf16Cvt::narrow2Q(x0 - __uint_as_float(hi << 16), x1 - __uint_as_float(hi & 0xFFFF0000u));
+    } else {
+        const v2h h = __builtin_convertvector(v2f{x0, x1}, v2h);
+        hi = __builtin_bit_cast(uint32_t, h);
+        lo = __builtin_bit_cast(uint32_t, __builtin_convertvector(v2f{x0 - float(h[0]), x1 - float(h[1])}, v2h));
+    }
+}
 
-    const size_t nqb = (a.seq + kMfmaQ - 1) / kMfmaQ;
+template <typename T>
+__device__ __forceinline__ f32x16 mfma32(const v4u &a, const v4u &b, const f32x16 &c) {
+    if constexpr (std::is_same_v<T, BF16>)
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(asBf16x8(a), asBf16x8(b), c, 0, 0, 0);
+    else
+        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+}
+
+// 16 INT8 codes -> T(code * sc) as 8 packed words (bf16: codesToBf16's exact product)
+template <typename T>
+__device__ __forceinline__ void codesToRow(const v4u &raw, float sc, v4u (&out)[2]) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const v4u half = h ? v4u{raw.z, raw.w, 0u, 0u} : v4u{raw.x, raw.y, 0u, 0u};
+        if constexpr (std::is_same_v<T, BF16>) {
+            out[h] = codesToBf16(half, sc);
+        } else {
+            float f[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) f[e] = float(int8_t(half[e / 4] >> (8 * (e % 4)))) * sc;
+            out[h] = Fmt<F16>::pack(f);
+        }
+    }
+}
+
+// Keys that the queries [q0, q1] see: the most and the fewest.  Where seq > total the first seq -
+// total queries wrap and see every key (visibleKeys).
+__device__ __forceinline__ void visibleRange(size_t total, size_t seq, size_t q0, size_t q1, size_t &most, size_t &least) {
+    const size_t wrapped = seq > total ? seq - total : 0;
+    most = q0 < wrapped ? total : visibleKeys(total, seq, q1);
+    least = q1 < wrapped ? total : visibleKeys(total, seq, q0 < wrapped ? wrapped : q0);
+}
+
+template <typename T, bool kInt8, int D, bool kHeads>
+__global__ void __launch_bounds__(kWave * 2 * kSplits, 2)
+    attnPrefill(AttnArgs a) {
+    constexpr int RB = 2 * D, C = RB / 16;       // bytes and chunks of a key row
+    constexpr int QS = D / 16, DT = D / 32;      // MFMA steps of q . k, column tiles of O
+    constexpr int kTileB = 32 * RB;              // one K or V tile of a wave's step
+    constexpr int kStageB = kSplits * 2 * kTileB; // [split][K tile | V tile]
+    constexpr int kLoads = kTileB / 1024;        // loads per wave: unit 0 the K tile, unit 1 the V tile
+    constexpr float kBias = std::is_same_v<T, F16> ? 8.0f : 0.0f; // base-2 exponent added to the weights
+    __shared__ __align__(16) char lds[2 * kStageB];
+    __shared__ float ml[2][kSplits][2][32];
+    const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) / kWave);
+    const int unit = wave / kSplits, split = wave % kSplits;
+    const int lane = int(threadIdx.x) % kWave;
+    const int n = lane % 32, h2 = lane / 32;
+
+    constexpr int kBlockQ = kHeads ? 32 : 64;
+    const size_t nqb = (a.seq + kBlockQ - 1) / kBlockQ;
     unsigned b = blockIdx.x;
+    const int c = int(b % unsigned(a.nchunks));
+    b /= unsigned(a.nchunks);
     const int sl = int(b % unsigned(a.slices));
     b /= unsigned(a.slices);
     const int g = int(b % unsigned(a.nkvh));
-    const size_t qb = nqb - 1 - size_t(b / unsigned(a.nkvh)); // latest queries first
-    const int h = g * a.group + sl * W + wave;
-    const size_t q0 = qb * kMfmaQ;
-    const size_t qi = min(q0 + size_t(n), a.seq - 1);
+    const size_t qb = nqb - 1 - size_t(b / unsigned(a.nkvh)); // latest queries (most keys) first
+    const int h = g * a.group + (kHeads ? 2 * sl + unit : sl);
+    const size_t q0 = qb * kBlockQ + (kHeads ? 0 : 32 * unit);
+    const size_t qi = min(q0 + size_t(n), a.seq - 1); // this lane's query (clamped for loads)
     const size_t vis_q = visibleKeys(a.total, a.seq, qi);
-    const size_t vis_blk = visibleKeys(a.total, a.seq, min(q0 + kMfmaQ - 1, a.seq - 1));
-    const size_t vis_first = visibleKeys(a.total, a.seq, q0);
-    const size_t ntiles = (vis_blk + kMfmaKT - 1) / kMfmaKT;
-    const float c2 = a.scale * 1.4426950408889634f;
+    size_t most, least;
+    visibleRange(a.total, a.seq, qb * kBlockQ, min(qb * kBlockQ + kBlockQ - 1, a.seq - 1), most, least);
+    const size_t k0 = size_t(c) * size_t(a.chunk); // a multiple of kStepKeys
+    const size_t k1 = a.nchunks == 1 ? most : min(most, k0 + size_t(a.chunk));
+    const int steps = k1 > k0 ? int((k1 - k0 + kStepKeys - 1) / kStepKeys) : 0;
+    const float c2 = a.scale * 1.4426950408889634f; // scores to base-2 exponents
 
-    bf16x8 qreg[KB];
+    v4u qreg[QS];
 #pragma unroll
-    for (int kb = 0; kb < KB; ++kb) {
-        const uint16_t *qp = static_cast<const uint16_t *>(a.q) + (qi * a.nh + h) * D + 32 * kb + 8 * g4;
-        qreg[kb] = asBf16x8(*reinterpret_cast<const v4u *>(qp));
-    }
-    float m = -INFINITY, lsum = 0.0f;
-    f32x4 o[DT];
+    for (int st = 0; st < QS; ++st)
+        qreg[st] = *reinterpret_cast<const v4u *>(static_cast<const uint16_t *>(a.q) + (qi * a.nh + h) * D + 16 * st + 8 * h2);
+    float m = -INFINITY, lsum = 0.0f; // m: running max of the raw dots (scaled by c2 in use)
+    f32x16 o[DT];
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt) o[dt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[dt][i] = 0.0f;
 
-    // load instruction j of this wave is stage load q = wave + W j (K rows for q < 16, then
-    // V rows): rows 4 (q % 16) + lane / 16 of the tile, LDS slot lane % 16 receiving chunk
-    // slot ^ swizzle(row) of the kv head's row
-    const size_t rowB = size_t(a.nkvh) * kRowB; // bytes between consecutive keys
-    const char *cache[2] = {static_cast<const char *>(a.k), static_cast<const char *>(a.v)};
-    // (byte offsets within a tile fit 32 bits: the launcher checks 64 rows * rowB < 2^31)
-    int lrow[kPer];
-    uint32_t loff[kPer], lcol[kPer];
+    const auto swzRow = [](bool v, int r) { // chunk XOR of row r of a tile
+        if (D == 128) return v ? 4 * (r & 3) : r & 15;
+        return v ? 4 * ((r >> 1) & 1) : (r >> 1) & 7;
+    };
+    // This wave's share of a step's loads: its split's K tile (unit 0) or V tile (unit 1).  Elements:
+    // load j fills 1 KB, rows j (1024 / RB) + lane / C.  Codes: lane l takes 16-code pieces l, l + 64, ...
+    const char *cache = static_cast<const char *>(unit ? a.v : a.k);
+    const float *cscale = unit ? a.vs : a.ks;
+    char *const mine = lds + split * 2 * kTileB + unit * kTileB;
+    constexpr int kCodeLoads = 32 * D / 16 / kWave;
+    v4u craw[kInt8 ? kCodeLoads : 1];
+    float csc[kInt8 ? kCodeLoads : 1];
+    const auto issue = [&](int step, int stage) {
+        const size_t t0 = k0 + size_t(step) * kStepKeys + size_t(32 * split);
+        if constexpr (kInt8) {
 #pragma unroll
-    for (int j = 0; j < kPer; ++j) {
-        const int q = wave + W * j;
-        const int row = 4 * (q % 16) + lane / 16, slot = lane % 16;
-        const int chunk = slot ^ (q < 16 ? swzK(row) : swzV(row));
-        lrow[j] = row;
-        lcol[j] = uint32_t(g * kRowB + chunk * 16);
-        loff[j] = uint32_t(row) * uint32_t(rowB) + lcol[j];
-    }
-    const auto issue = [&](size_t t0, int stage) {
-        char *dst = &lds_all[half][stage][0];
-        const size_t left = a.total - t0; // keys of the cache from t0 on (> 0)
-        const bool full = left >= size_t(kMfmaKT);
+            for (int j = 0; j < kCodeLoads; ++j) {
+                const int piece = lane + kWave * j, row = piece / (D / 16), col = 16 * (piece % (D / 16));
+                const size_t key = (t0 + row < a.total ? t0 + row : 0) * size_t(a.nkvh) + size_t(g);
+                const v2u lo = *reinterpret_cast<const v2u *>(cache + key * D + col); // 8-byte aligned codes
+                const v2u hi = *reinterpret_cast<const v2u *>(cache + key * D + col + 8);
+                craw[j] = v4u{lo.x, lo.y, hi.x, hi.y};
+                csc[j] = cscale[key];
+            }
+        } else {
 #pragma unroll
-        for (int j = 0; j < kPer; ++j) {
-            const int q = wave + W * j;
-            if (q >= kLoads) break;
-            // the tile's rows from the tile base; in the cache's last tile, rows past it read row 0
-            const char *src = full || size_t(lrow[j]) < left ? cache[q / 16] + t0 * rowB + loff[j]
-                                                            : cache[q / 16] + lcol[j];
-            __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1))) *)(src),
-                                             (void __attribute__((address_space(3))) *)(dst + q * 1024), 16, 0, 0);
+            for (int j = 0; j < kLoads; ++j) {
+                const int row = j * (1024 / RB) + lane / C, chunk = (lane % C) ^ swzRow(unit, row);
+                const size_t key = (t0 + row < a.total ? t0 + row : 0) * size_t(a.nkvh) + size_t(g);
+                __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1))) *)(cache + key * RB + 16 * chunk),
+                                                 (void __attribute__((address_space(3))) *)(mine + stage * kStageB + j * 1024), 16, 0, 0);
+            }
+        }
+    };
+    const auto land = [&](int stage) { // the loads issued last are in LDS (this wave's)
+        if constexpr (kInt8) {
+#pragma unroll
+            for (int j = 0; j < kCodeLoads; ++j) {
+                const int piece = lane + kWave * j, row = piece / (D / 16), col = 2 * (piece % (D / 16));
+                v4u el[2];
+                codesToRow<T>(craw[j], csc[j], el);
+#pragma unroll
+                for (int e = 0; e < 2; ++e)
+                    *reinterpret_cast<v4u *>(mine + stage * kStageB + row * RB + 16 * ((col + e) ^ swzRow(unit, row))) = el[e];
+            }
+        } else {
+            waitVmcnt<0>();
         }
     };
 
-    const size_t nsteps = kSplit ? (ntiles + 1) / 2 : ntiles;
-    const size_t tbeg = half ? nsteps : 0;
-    const size_t tcount = half ? ntiles - nsteps : nsteps;
-    if (tcount > 0) issue(tbeg * kMfmaKT, 0);
-    for (size_t it = 0; it < nsteps; ++it) {
-        const int buf = int(it & 1);
-        const size_t kt0 = (tbeg + it) * kMfmaKT;
-        waitVmcnt<0>(); // this wave's loads of tile it have landed
-        ldsBarrier();   // every wave's have; every wave is past the step that read the other stage
-        if (it + 1 < tcount) issue(kt0 + kMfmaKT, buf ^ 1);
-        if (kSplit && it >= tcount) continue;
-        const char *kt = &lds_all[half][buf][0], *vt = kt + kTileB;
-        const bool whole = kt0 + kMfmaKT <= vis_first;
-        const int nvis = int(min(vis_q - min(vis_q, kt0), size_t(kMfmaKT)));
-        float p[4][4];
+    // this lane's K row (A row n) and V row pieces within a tile
+    const int krow = 16 * (n / 16) + 8 * ((n >> 2) & 1) + 4 * ((n >> 3) & 1) + n % 4;
+    const int ksw = swzRow(false, krow);
+    const int vrow = 8 * h2 + (lane % 16) / 4; // and + 4, + 16
+    if (steps > 0) issue(0, 0);
+    for (int it = 0; it < steps; ++it) {
+        const int buf = it & 1;
+        land(buf);
+        ldsBarrier(); // every wave's tiles of this step are in LDS, and the other stage is no longer read
+        if (it + 1 < steps) issue(it + 1, buf ^ 1);
+        const size_t kt0 = k0 + size_t(it) * kStepKeys + size_t(32 * split);
+        if (kt0 >= k1) continue; // the last step may not reach this split
+        const char *kt = lds + buf * kStageB + split * 2 * kTileB, *vt = kt + kTileB;
+        f32x16 s;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s[i] = 0.0f;
+#pragma unroll
+        for (int st = 0; st < QS; ++st)
+            s = mfma32<T>(*reinterpret_cast<const v4u *>(kt + krow * RB + 16 * ((2 * st + h2) ^ ksw)), qreg[st], s);
+        if (kt0 + 32 > least) { // the causal diagonal or the cache's end (block-uniform): mask
+            const int nvis = int(min(vis_q - min(vis_q, kt0), size_t(32)));
+#pragma unroll
+            for (int i = 0; i < 16; ++i) s[i] = 16 * (i / 8) + 8 * h2 + i % 8 < nvis ? s[i] : -INFINITY;
+        }
         float mx = m;
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            const int krow = 32 * (t / 2) + 8 * (n / 4) + 4 * (t % 2) + n % 4; // A row n
-            const char *kr = kt + krow * kRowB;
-            const int sw = swzK(krow);
-            f32x4 acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int kb = 0; kb < KB; ++kb) {
-                const v4u kv = *reinterpret_cast<const v4u *>(kr + 16 * ((4 * kb + g4) ^ sw));
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(asBf16x8(kv), qreg[kb], acc, 0, 0, 0);
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i) p[t][i] = acc[i];
-        }
-        if (!whole) {
-#pragma unroll
-            for (int t = 0; t < 4; ++t)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int off = 32 * (t / 2) + 8 * g4 + 4 * (t % 2) + i;
-                    p[t][i] = off < nvis ? p[t][i] : -INFINITY;
-                }
-        }
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) mx = fmaxf(mx, p[t][i]);
-        mx = fmaxf(mx, __shfl_xor(mx, 16, kWave));
+        for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[i]);
         mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
-        const float mc = mx == -INFINITY ? 0.0f : mx * c2;
+        // exp(scale (s - max)) as 2^(s c2 - max c2); a masked key (-inf) gets weight 0: mc = 0 while
+        // every score is -inf keeps it 0 rather than NaN, with no per-score select
+        const float mc = (mx == -INFINITY ? 0.0f : mx * c2) - kBias;
         float ps = 0.0f;
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                p[t][i] = __builtin_amdgcn_exp2f(__builtin_fmaf(p[t][i], c2, -mc));
-                ps += p[t][i];
-            }
-        if (__builtin_expect(__any(mx != m), 0)) {
-            const float corr = mx == m ? 1.0f : __builtin_amdgcn_exp2f(__builtin_fmaf(m, c2, -mc));
+        for (int i = 0; i < 16; ++i) {
+            s[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], c2, -mc));
+            ps += s[i];
+        }
+        if (__builtin_expect(__any(mx != m), 0)) { // rescale only when a max moved
+            const float corr = mx == m ? 1.0f : __builtin_amdgcn_exp2f(__builtin_fmaf(m, c2, -mc - kBias));
             lsum *= corr;
 #pragma unroll
             for (int dt = 0; dt < DT; ++dt) o[dt] *= corr;
         }
         m = mx;
         lsum += ps;
-        // the transposing reads' rows and column offset: keys 32 p2 + 8 g + n / 4 (and + 4),
-        // columns 16 dt + 4 (n % 4) .. + 3, i.e. half n % 2 of chunk 2 dt + (n % 4) / 2
 #pragma unroll
-        for (int p2 = 0; p2 < 2; ++p2) {
+        for (int kg = 0; kg < 2; ++kg) {
             uint32_t hw[4], lw[4];
 #pragma unroll
-            for (int w = 0; w < 4; ++w) {
-                const float x0 = p[2 * p2 + w / 2][2 * (w % 2)], x1 = p[2 * p2 + w / 2][2 * (w % 2) + 1];
-                hw[w] = Bf16Cvt::narrow2Q(x0, x1);
-                lw[w] = Bf16Cvt::narrow2Q(x0 - __uint_as_float(hw[w] << 16), x1 - __uint_as_float(hw[w] & 0xFFFF0000u));
-            }
-            const bf16x8 bhi = asBf16x8(v4u{hw[0], hw[1], hw[2], hw[3]});
-            const bf16x8 blo = asBf16x8(v4u{lw[0], lw[1], lw[2], lw[3]});
-            const int r0 = 32 * p2 + 8 * g4 + n / 4;
-            const char *v0 = vt + r0 * kRowB + 8 * (n % 2), *v1 = v0 + 4 * kRowB;
-            const int sw = swzV(r0); // rows r0 and r0 + 4 share it
+            for (int w = 0; w < 4; ++w) splitPair<T>(s[8 * kg + 2 * w], s[8 * kg + 2 * w + 1], hw[w], lw[w]);
+            const v4u phi = {hw[0], hw[1], hw[2], hw[3]}, plo = {lw[0], lw[1], lw[2], lw[3]};
+            const int r0 = 16 * kg + vrow, r1 = r0 + 4;
+            const char *v0 = vt + r0 * RB + 8 * (lane % 2), *v1 = vt + r1 * RB + 8 * (lane % 2);
+            const int s0 = swzRow(true, r0), s1 = swzRow(true, r1);
 #pragma unroll
             for (int dt = 0; dt < DT; ++dt) {
-                const int cofs = 16 * ((2 * dt + (n % 4) / 2) ^ sw);
-                const uint64_t e0 = ldsReadTr16(v0 + cofs), e1 = ldsReadTr16(v1 + cofs);
-                const v4u vv = v4u{uint32_t(e0), uint32_t(e0 >> 32), uint32_t(e1), uint32_t(e1 >> 32)};
-                o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(asBf16x8(vv), bhi, o[dt], 0, 0, 0);
-                o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(asBf16x8(vv), blo, o[dt], 0, 0, 0);
+                // columns 32 dt + 16 (lane / 16 % 2) + 4 (lane % 4) ..: half lane % 2 of a chunk
+                const int ch = 4 * dt + 2 * (lane / 16 % 2) + (lane % 4) / 2;
+                const uint64_t e0 = ldsReadTr16(v0 + 16 * (ch ^ s0)), e1 = ldsReadTr16(v1 + 16 * (ch ^ s1));
+                const v4u vv = {uint32_t(e0), uint32_t(e0 >> 32), uint32_t(e1), uint32_t(e1 >> 32)};
+                o[dt] = mfma32<T>(vv, phi, o[dt]);
+                o[dt] = mfma32<T>(vv, plo, o[dt]);
             }
         }
     }
-    float lt = lsum + __shfl_xor(lsum, 16, kWave);
-    lt += __shfl_xor(lt, 32, kWave);
-    if constexpr (kSplit) {
-        float *xch = reinterpret_cast<float *>(&lds_all[0][0][0]) + size_t(wave) * kWave * (2 + 4 * DT);
-        __syncthreads();
-        if (half == 1) {
-            xch[lane] = m;
-            xch[kWave + lane] = lt;
-#pragma unroll
-            for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) xch[(2 + 4 * dt + i) * kWave + lane] = o[dt][i];
-        }
-        __syncthreads();
-        if (half == 1) return;
-        const float m1 = xch[lane], l1 = xch[kWave + lane];
-        const float M = fmaxf(m, m1);
-        const float f0 = m == M ? 1.0f : __builtin_amdgcn_exp2f(__builtin_fmaf(m, c2, -M * c2));
-        const float f1 = m1 == M ? 1.0f : __builtin_amdgcn_exp2f(__builtin_fmaf(m1, c2, -M * c2));
-        lt = lt * f0 + l1 * f1;
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) o[dt][i] = o[dt][i] * f0 + xch[(2 + 4 * dt + i) * kWave + lane] * f1;
+    lsum += __shfl_xor(lsum, 32, kWave);
+
+    // merge the splits: every wave leaves (max, sum, output) in LDS, then wave (u, s) finishes the
+    // column tiles s, s + kSplits, .. of unit u
+    ldsBarrier(); // the tiles are no longer read
+    float *const xo = reinterpret_cast<float *>(lds); // [unit][split][dt][i / 4][lane][4]
+    static_assert(2 * kSplits * DT * 16 * kWave * 4 <= 2 * kStageB, "the outputs fit the tiles' storage");
+    if (h2 == 0) {
+        ml[unit][split][0][n] = m;
+        ml[unit][split][1][n] = lsum;
     }
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            *reinterpret_cast<f32x4 *>(xo + ((((unit * kSplits + split) * DT + dt) * 4 + q) * kWave + lane) * 4) =
+                f32x4{o[dt][4 * q], o[dt][4 * q + 1], o[dt][4 * q + 2], o[dt][4 * q + 3]};
+    ldsBarrier();
     if (q0 + size_t(n) >= a.seq) return;
-    const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
-    uint16_t *op = static_cast<uint16_t *>(a.out) + (qi * a.nh + h) * D + 4 * g4;
+    float M = -INFINITY, L = 0.0f, f[kSplits];
+#pragma unroll
+    for (int k = 0; k < kSplits; ++k) M = fmaxf(M, ml[unit][k][0][n]);
+#pragma unroll
+    for (int k = 0; k < kSplits; ++k) {
+        const float mk = ml[unit][k][0][n];
+        f[k] = mk == M ? 1.0f : __builtin_amdgcn_exp2f((mk - M) * c2); // 1 for M = -inf, where l = o = 0
+        L += ml[unit][k][1][n] * f[k];
+    }
+    const size_t ih = qi * a.nh + size_t(h);
+    float *const part = a.nchunks > 1 ? a.part + (ih * size_t(a.nchunks) + c) * (D + 2) : nullptr;
+    const float inv = L > 0.0f ? 1.0f / L : 0.0f;
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) {
-        const uint32_t w0 = f32ToBf16(o[dt][0] * inv) | (f32ToBf16(o[dt][1] * inv) << 16);
-        const uint32_t w1 = f32ToBf16(o[dt][2] * inv) | (f32ToBf16(o[dt][3] * inv) << 16);
-        typedef uint32_t v2u __attribute__((ext_vector_type(2)));
-        *reinterpret_cast<v2u *>(op + 16 * dt) = v2u{w0, w1};
+        if (dt % kSplits != split) continue;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            f32x4 O = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int k = 0; k < kSplits; ++k)
+                O += f[k] * *reinterpret_cast<const f32x4 *>(xo + ((((unit * kSplits + k) * DT + dt) * 4 + q) * kWave + lane) * 4);
+            const int col = 32 * dt + 8 * q + 4 * h2;
+            if (part) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) part[col + e] = O[e];
+            } else {
+                using Cv = std::conditional_t<std::is_same_v<T, BF16>, Bf16Cvt, F16Cvt>; // the reference rounding
+                *reinterpret_cast<v2u *>(static_cast<uint16_t *>(a.out) + ih * D + col) =
+                    v2u{Cv::narrow(O[0] * inv) | (Cv::narrow(O[1] * inv) << 16), Cv::narrow(O[2] * inv) | (Cv::narrow(O[3] * inv) << 16)};
+            }
+        }
     }
+    if (part && split == 0 && h2 == 0) {
+        part[D] = M * a.scale; // the scaled units attnCombine works in
+        part[D + 1] = L;
+    }
+}
+
+// Merge of few chunk partials for many (query, head) pairs: a thread per 4 columns of a pair.
+// (attnCombine spends 1024 threads on 32 columns of a pair, for up to 1024 chunks.)
+template <typename T>
+__global__ void __launch_bounds__(256)
+    attnCombineFew(void *out, const float *part, int nchunks, int D, size_t pairs) {
+    const size_t idx = size_t(blockIdx.x) * 256 + threadIdx.x;
+    const int per = D / 4;
+    const size_t ih = idx / per;
+    if (ih >= pairs) return;
+    const int col = 4 * int(idx % per);
+    const float *pp = part + ih * size_t(nchunks) * (D + 2);
+    float M = -INFINITY, L = 0.0f, O[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int c = 0; c < nchunks; ++c) M = fmaxf(M, pp[size_t(c) * (D + 2) + D]);
+    for (int c = 0; c < nchunks; ++c) {
+        const float *pc = pp + size_t(c) * (D + 2);
+        const float f = pc[D] == M ? 1.0f : __expf(pc[D] - M); // 1 for M = -inf, where l = o = 0
+        L += pc[D + 1] * f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) O[e] += pc[col + e] * f;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) Fmt<T>::put(out, ih * D + col + e, L > 0.0f ? O[e] / L : 0.0f);
 }
 
 // ---- decode on MFMA (bf16 q / out, head_dim 128, cache in bf16 or INT8) ---------------
@@ -1175,13 +1011,54 @@ bool vecShape(const AttnArgs &a, int d, int dv, bool int8) {
            (int8 ? aligned(a.k, 8) && aligned(a.v, 8) : aligned(a.k, 16) && aligned(a.v, 16));
 }
 
-// The bf16 prefill on MFMA: head_dim 128, 16 or more queries, a non-empty cache and a
-// positive finite scale (the kernel tracks the max of the raw dot products).
-bool prefillMfma(const AttnArgs &a, int d, int dv, bool int8, bool bf16) {
-    if (!bf16 || !vecShape(a, d, dv, int8)) return false;
-    const size_t mblocks = (a.seq + kMfmaQ - 1) / kMfmaQ * size_t(a.nkvh) * size_t(a.group / sliceOf(a.group));
-    return d == 128 && a.total > 0 && a.seq >= size_t(kMfmaQ) && mblocks < (size_t(1) << 31) &&
-           a.scale > 0.0f && std::isfinite(a.scale);
+// The prefill on MFMA: bf16 or f16, head_dim 64 or 128, 16 or more queries, a non-empty cache and
+// a positive finite scale (the kernel tracks the max of the raw dot products).
+struct Prefill {
+    int slices, chunk, nchunks;
+    size_t blocks, part_bytes;
+    bool heads; // the block's units are two q heads (else two 32-query blocks of one head)
+};
+constexpr size_t kPrefillPartBytes = size_t(8) << 20;
+
+// How the prefill is cut; false where it does not apply.  Depends on the shape only, so that every
+// entry point sums a shape in the same order.  Keys are split over blocks where the query blocks
+// alone would leave CUs idle, into chunks of at least 4 steps (512 keys): 16 queries over 32768
+// keys would otherwise be 256 steps in each of 6 blocks.
+bool planPrefill(Prefill &p, const AttnArgs &a, int d, int dv, bool int8, llaisysDataType_t dt) {
+    if ((dt != LLAISYS_DTYPE_BF16 && dt != LLAISYS_DTYPE_F16) || !vecShape(a, d, dv, int8)) return false;
+    if (a.total == 0 || a.seq < size_t(kMfmaQ) || !(a.scale > 0.0f) || !std::isfinite(a.scale)) return false;
+    p.heads = a.group % 2 == 0;
+    p.slices = p.heads ? a.group / 2 : a.group;
+    const size_t qb = (a.seq + (p.heads ? 31 : 63)) / (p.heads ? 32 : 64);
+    p.blocks = qb * size_t(a.nkvh) * size_t(p.slices);
+    const size_t steps = (a.total + kStepKeys - 1) / kStepKeys;
+    const size_t cap = kPrefillPartBytes / (a.seq * size_t(a.nh) * size_t(d + 2) * sizeof(float));
+    size_t n = std::max<size_t>(1, std::min({256 / p.blocks, steps / 4, cap, size_t(1024)}));
+    const size_t per = (steps + n - 1) / n;
+    n = (steps + per - 1) / per;
+    if (per * kStepKeys > size_t(INT32_MAX)) return false;
+    p.chunk = int(per * kStepKeys);
+    p.nchunks = int(n);
+    p.part_bytes = n > 1 ? a.seq * size_t(a.nh) * n * size_t(d + 2) * sizeof(float) : 0;
+    p.blocks *= n;
+    return p.blocks < (size_t(1) << 31);
+}
+
+template <typename T, bool kInt8>
+void launchPrefill(const AttnArgs &a, const Prefill &p, int d, hipStream_t s) {
+    const unsigned blocks = unsigned(p.blocks), threads = kWave * 2 * kSplits;
+    if (d == 128)
+        p.heads ? attnPrefill<T, kInt8, 128, true><<<blocks, threads, 0, s>>>(a)
+                : attnPrefill<T, kInt8, 128, false><<<blocks, threads, 0, s>>>(a);
+    else
+        p.heads ? attnPrefill<T, kInt8, 64, true><<<blocks, threads, 0, s>>>(a)
+                : attnPrefill<T, kInt8, 64, false><<<blocks, threads, 0, s>>>(a);
+    if (p.nchunks == 1) return;
+    const size_t pairs = a.seq * size_t(a.nh);
+    if (p.nchunks <= 16)
+        attnCombineFew<T><<<unsigned((pairs * size_t(d / 4) + 255) / 256), 256, 0, s>>>(a.out, a.part, p.nchunks, d, pairs);
+    else
+        launchCombine<T>(a.out, a.part, p.nchunks, d, pairs, s);
 }
 
 template <typename T, bool kInt8>
@@ -1195,67 +1072,30 @@ void launch(AttnArgs a, int d, int dv, void *ws, size_t ws_bytes, hipStream_t s)
     }
     const int G = sliceOf(a.group);
     a.slices = a.group / G;
-    // bf16 prefill (16 or more queries, cache in bf16 or INT8) goes to the MFMA kernel;
-    // decode and the other types stay on the vector kernel
-    if constexpr (std::is_same_v<T, BF16>) {
-        const size_t mblocks = (a.seq + kMfmaQ - 1) / kMfmaQ * size_t(a.nkvh) * size_t(a.slices);
-        if (prefillMfma(a, d, dv, kInt8, true)) {
-            a.nchunks = 1;
+    if constexpr (!std::is_same_v<T, F32>) {
+        constexpr auto dt = std::is_same_v<T, BF16> ? LLAISYS_DTYPE_BF16 : LLAISYS_DTYPE_F16;
+        Prefill p;
+        if (planPrefill(p, a, d, dv, kInt8, dt) && p.part_bytes <= ws_bytes) {
+            a.slices = p.slices;
+            a.chunk = p.chunk;
+            a.nchunks = p.nchunks;
+            a.part = static_cast<float *>(ws);
             if constexpr (kInt8) {
-                // An INT8 cache whose bf16 form fits the workspace is dequantized once (both
-                // caches in one launch, bf16(code * scale) as the tiles would be staged) and
-                // attended as bf16: the tile staging of every query block no longer converts
-                // the same codes again.  Same operands, so the same bits.
-                const size_t cache_el = a.total * size_t(a.nkvh) * size_t(d);
-                if (2 * cache_el * sizeof(uint16_t) <= ws_bytes) {
-                    uint16_t *kd = static_cast<uint16_t *>(ws), *vd = kd + cache_el;
+                // An INT8 cache whose 16-bit form fits the workspace behind the partials is
+                // dequantized once (both caches in one launch, T(code * scale) as the tiles would be
+                // staged), so that the tiles of every query block no longer convert the same codes.
+                const size_t cache_el = a.total * size_t(a.nkvh) * size_t(d), off = (p.part_bytes + 255) / 256 * 256;
+                if (off + 2 * cache_el * sizeof(uint16_t) <= ws_bytes) {
+                    uint16_t *kd = reinterpret_cast<uint16_t *>(static_cast<char *>(ws) + off), *vd = kd + cache_el;
                     dequantizeInt8Pair(kd, static_cast<const int8_t *>(a.k), a.ks, a.total * size_t(a.nkvh), vd,
                                        static_cast<const int8_t *>(a.v), a.vs, a.total * size_t(a.nkvh),
-                                       size_t(d), LLAISYS_DTYPE_BF16, s);
-                    AttnArgs b = a;
-                    b.k = kd;
-                    b.v = vd;
-                    b.ks = b.vs = nullptr;
-                    return launch<T, false>(b, d, dv, nullptr, 0, s);
+                                       size_t(d), dt, s);
+                    a.k = kd;
+                    a.v = vd;
+                    return launchPrefill<T, false>(a, p, d, s);
                 }
             }
-            // few blocks per CU: the causal imbalance is not averaged out across blocks, so
-            // the key tiles of each block are split over two wave sets
-            // (groups of 8 keep one wave per head: 16 waves of 8 heads would spill registers).
-            // A bf16 cache's tiles go HBM -> LDS directly (attnMfmaLds; its byte offsets
-            // within a tile take 32 bits, so beyond 2^17 kv heads the register-staged kernel).
-            if (!kInt8 && size_t(a.nkvh) * 256 * kMfmaKT < (size_t(1) << 31)) {
-                if (mblocks <= 512 && G <= 6) {
-                    switch (G) {
-                    case 6: attnMfmaLds<6, true><<<unsigned(mblocks), kWave * 12, 0, s>>>(a); return;
-                    case 4: attnMfmaLds<4, true><<<unsigned(mblocks), kWave * 8, 0, s>>>(a); return;
-                    case 2: attnMfmaLds<2, true><<<unsigned(mblocks), kWave * 4, 0, s>>>(a); return;
-                    default: attnMfmaLds<1, true><<<unsigned(mblocks), kWave * 2, 0, s>>>(a); return;
-                    }
-                }
-                switch (G) {
-                case 8: attnMfmaLds<8, false><<<unsigned(mblocks), kWave * 8, 0, s>>>(a); return;
-                case 6: attnMfmaLds<6, false><<<unsigned(mblocks), kWave * 6, 0, s>>>(a); return;
-                case 4: attnMfmaLds<4, false><<<unsigned(mblocks), kWave * 4, 0, s>>>(a); return;
-                case 2: attnMfmaLds<2, false><<<unsigned(mblocks), kWave * 2, 0, s>>>(a); return;
-                default: attnMfmaLds<1, false><<<unsigned(mblocks), kWave, 0, s>>>(a); return;
-                }
-            }
-            if (mblocks <= 512 && G <= 6) {
-                switch (G) {
-                case 6: attnMfma<6, true, kInt8><<<unsigned(mblocks), kWave * 12, 0, s>>>(a); return;
-                case 4: attnMfma<4, true, kInt8><<<unsigned(mblocks), kWave * 8, 0, s>>>(a); return;
-                case 2: attnMfma<2, true, kInt8><<<unsigned(mblocks), kWave * 4, 0, s>>>(a); return;
-                default: attnMfma<1, true, kInt8><<<unsigned(mblocks), kWave * 2, 0, s>>>(a); return;
-                }
-            }
-            switch (G) {
-            case 8: attnMfma<8, false, kInt8><<<unsigned(mblocks), kWave * 8, 0, s>>>(a); return;
-            case 6: attnMfma<6, false, kInt8><<<unsigned(mblocks), kWave * 6, 0, s>>>(a); return;
-            case 4: attnMfma<4, false, kInt8><<<unsigned(mblocks), kWave * 4, 0, s>>>(a); return;
-            case 2: attnMfma<2, false, kInt8><<<unsigned(mblocks), kWave * 2, 0, s>>>(a); return;
-            default: attnMfma<1, false, kInt8><<<unsigned(mblocks), kWave, 0, s>>>(a); return;
-            }
+            return launchPrefill<T, kInt8>(a, p, d, s);
         }
     }
     // bf16 decode (fewer than 16 queries): the MFMA decode kernel, one 32-key step per wave
@@ -1369,9 +1209,10 @@ size_t selfAttentionInt8KVScratchBytes(const void *out, const void *q, const voi
     a.nkvh = int(nkvh);
     a.group = int(nh / nkvh);
     a.scale = scale;
-    if (seq > 0 && nh > 0 && prefillMfma(a, int(d), int(dv), true, dt == LLAISYS_DTYPE_BF16)) {
-        const size_t cache = 2 * total * nkvh * d * sizeof(uint16_t);
-        return cache <= cap ? cache : 0;
+    Prefill p;
+    if (seq > 0 && nh > 0 && dt == LLAISYS_DTYPE_BF16 && d == 128 && planPrefill(p, a, int(d), int(dv), true, dt)) {
+        const size_t part = (p.part_bytes + 255) / 256 * 256, cache = 2 * total * nkvh * d * sizeof(uint16_t);
+        return part + cache <= cap ? part + cache : part;
     }
     return selfAttentionWorkspaceBytes(seq, nh, d);
 }

@@ -1,0 +1,71 @@
+"""The MFMA prefill attention (attnPrefill) at the edges of its tiles, against the oracle: both
+16-bit types, both head dims, cache in the type and in INT8.  Tolerance: assert_attention_close."""
+import zlib
+
+import numpy as np
+import pytest
+
+import llaisys_amd as L
+import oracle
+from numerics import assert_attention_close, assert_exact
+from test_attention_gpu import AMD, DTS, attend, dev, sample
+
+pytestmark = pytest.mark.gpu
+
+# seq, total, nh, nkvh, d: one query block, one key over a step of 128 and over a split of 32, the last
+# query block of one query, even and odd groups (two heads / two query blocks per block), keys split
+# over blocks (few and many chunks), more queries than keys (the early ones wrap and see every key)
+EDGES = [(16, 16, 2, 1, 64), (33, 129, 4, 2, 128), (64, 97, 3, 1, 64), (65, 160, 5, 5, 128), (97, 384, 12, 2, 64),
+         (16, 4100, 12, 2, 128), (31, 20000, 3, 3, 64), (300, 200, 4, 2, 128), (130, 100, 3, 1, 64)]
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("shape", EDGES, ids=lambda s: "x".join(map(str, s)))
+def test_prefill_tiles(dt, shape):
+    seq, total, nh, nkvh, d = shape
+    rng = np.random.default_rng(zlib.crc32(repr((dt, shape)).encode()))
+    q, k, v = sample(rng, (seq, nh, d), dt), sample(rng, (total, nkvh, d), dt), sample(rng, (total, nkvh, d), dt)
+    scale = 1.0 / np.sqrt(d)
+    got = attend(q, k, v, scale, dt)
+    assert_attention_close(got, oracle.self_attention(q, k, v, scale), v, f"{dt} {shape}")
+    assert_exact(attend(q, k, v, scale, dt), got, "repeat")
+    # INT8: dequantized into the workspace, or converted in the tiles: the bits of the composition
+    (kq, ks), (vq, vs) = oracle.quantize_int8(k), oracle.quantize_int8(v)
+    tq, t8 = dev(q, DTS[dt]), [dev(a) for a in (kq, ks, vq, vs)]
+    out, ref = (L.Tensor((seq, nh, d), DTS[dt], **AMD) for _ in range(2))
+    L.Ops.self_attention_int8kv(out, tq, *t8, scale)
+    kd, vd = (L.Tensor((total, nkvh, d), DTS[dt], **AMD) for _ in range(2))
+    L.Ops.dequantize_int8_pair(kd, t8[0], t8[1], vd, t8[2], t8[3])
+    L.Ops.self_attention(ref, tq, kd, vd, scale)
+    assert_exact(out.numpy(), ref.numpy(), "int8 vs dequantize + attend")
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+def test_small_weights_keep_their_share(dt):
+    """One key with nearly all of the weight and many with 2^-15 of it each: their sum still counts
+    (the weights enter the matrix product as two 16-bit parts)."""
+    d, total = 64, 1024
+    rng = np.random.default_rng(3)
+    q = np.zeros((16, 2, d), np.float32)
+    q[..., 0] = 1.0
+    k = np.zeros((total, 1, d), np.float32)
+    k[0, 0, 0] = 15 * np.log(2)
+    v = (1 + rng.random((total, 1, d))).astype(np.float32)
+    to = {"bf16": lambda x: (x.view(np.uint32) >> 16).astype(np.uint16), "f16": lambda x: x.astype(np.float16)}[dt]
+    q, k, v = to(q), to(k), to(v)
+    got = attend(q, k, v, 1.0, dt)
+    assert_attention_close(got, oracle.self_attention(q, k, v, 1.0), v, dt)
+
+
+def test_no_alloc_prefill_over_a_split_cache():
+    """Keys split over blocks, the caches too large for the fixed scratch beside the partials: the
+    codes are converted in the tiles, with the bits of the allocating entry point."""
+    seq, total, nh, nkvh, d = 40, 30000, 12, 2, 128
+    rng = np.random.default_rng(9)
+    q, k, v = sample(rng, (seq, nh, d), "bf16"), sample(rng, (total, nkvh, d), "bf16"), sample(rng, (total, nkvh, d), "bf16")
+    (kq, ks), (vq, vs) = oracle.quantize_int8(k), oracle.quantize_int8(v)
+    tq, t8 = dev(q, DTS["bf16"]), [dev(a) for a in (kq, ks, vq, vs)]
+    out, ref = (L.Tensor((seq, nh, d), DTS["bf16"], **AMD) for _ in range(2))
+    L.Ops.self_attention_int8kv(ref, tq, *t8, 0.0883883)
+    L.Ops.self_attention_int8kv_noalloc(out, tq, *t8, 0.0883883)
+    assert_exact(out.numpy(), ref.numpy(), "no alloc")
