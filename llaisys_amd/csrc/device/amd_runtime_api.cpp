@@ -234,11 +234,14 @@ void *tryWorkspace(int dev, size_t bytes, llaisysStream_t s) {
     CHECK_ARGUMENT(dev >= 0 && dev < kMaxDevices, "device id out of range");
     WsSlots &ws = wsSlots();
     std::shared_ptr<WsBuffer> &cur = ws.buf[dev];
+    if (!ws.capturing[dev]) {
+        // a graph that the caller captures on the stream itself does not keep the buffer alive
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(static_cast<hipStream_t>(s), &cap) != hipSuccess || cap != hipStreamCaptureStatusNone)
+            return nullptr;
+    }
     if (cur && cur->size >= bytes) return cur->ptr;
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (ws.capturing[dev] || hipStreamIsCapturing(static_cast<hipStream_t>(s), &cap) != hipSuccess ||
-        cap != hipStreamCaptureStatusNone)
-        return nullptr;
+    if (ws.capturing[dev]) return nullptr;
     const char *what = nullptr;
     if (growWorkspace(cur, bytes, what) != hipSuccess) {
         (void)hipGetLastError(); // the caller goes on without: leave no sticky error

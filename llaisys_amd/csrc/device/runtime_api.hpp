@@ -29,9 +29,9 @@ void raiseIfError(llaisysStream_t stream);
 // least `bytes` of device memory, zeroed when first allocated.  A growth moves the thread
 // to a new buffer; the old one is freed once no captured graph holds it.
 void *workspace(int device_id, size_t bytes);
-// The same scratch for a caller that can do without: null where it would have to grow while
-// `stream` is being captured (by llaisysGraphBeginCapture or by the caller itself), or where the
-// memory is not there.
+// The same scratch for an op that can do without: null where it would have to grow during
+// llaisysGraphBeginCapture, where `stream` is being captured by other means (such a graph does not
+// keep the scratch alive), or where the memory is not there.
 void *tryWorkspace(int device_id, size_t bytes, llaisysStream_t stream);
 
 // HIP-graph capture of the work enqueued on `stream` (the current device's context stream).

@@ -57,11 +57,13 @@ void embedding(void *out, const void *index, bool index_i64, size_t n_index, con
                size_t vocab, size_t row_bytes, int *err, hipStream_t stream);
 
 // Per-row argmax of vals [rows, cols]; idx is I32 or I64, val has the dtype of vals.
+// With `workspace` (the library scratch, >= kScratchReserved bytes) few rows are spread over more
+// blocks than one each; without it they are not.
 void argmaxRows(void *idx, bool idx_i64, void *val, const void *vals, size_t rows, size_t cols,
-                llaisysDataType_t dt, hipStream_t stream);
+                llaisysDataType_t dt, void *workspace, hipStream_t stream);
 
 // Library scratch layout (zeroed once when allocated): bytes [0, 256) hold the flat argmax's
-// completion counter and [kSampleStateOffset, kScratchReserved) the sampler's per-row
+// completion counter and key (16 of them, one per row of a few-row argmax) and [kSampleStateOffset, kScratchReserved) the sampler's per-row
 // histograms and counters; both stay zero between launches.  Other users of the scratch
 // start at kScratchReserved.
 constexpr size_t kSampleRows = 16;            // rows per sampler launch

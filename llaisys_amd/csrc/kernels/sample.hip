@@ -492,7 +492,7 @@ void randomSample(void *out_idx, bool i64, const void *logits, size_t rows, size
         if (rows == 1) // one row: the multi-block flat argmax (its workspace: base, counter at 0)
             argmax(out_idx, i64, val, logits, V, dt, base, s);
         else
-            argmaxRows(out_idx, i64, val, logits, rows, V, dt, s);
+            argmaxRows(out_idx, i64, val, logits, rows, V, dt, base, s);
         return;
     }
     const float inv = 1.0f / temperature;

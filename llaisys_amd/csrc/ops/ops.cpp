@@ -91,7 +91,8 @@ void argmaxRows(tensor_t max_idx, tensor_t max_val, tensor_t vals) {
            "ArgmaxRows: outputs must hold one element per row");
     auto s = streamFor(vals);
     kernels::argmaxRows(max_idx->data(), max_idx->dtype() == LLAISYS_DTYPE_I64, max_val->data(),
-                        vals->data(), rows, cols, vals->dtype(), s);
+                        vals->data(), rows, cols, vals->dtype(),
+                        device::amd::tryWorkspace(vals->deviceId(), kernels::kScratchReserved, s), s);
     launched("argmaxRows");
 }
 

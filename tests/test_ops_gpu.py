@@ -981,3 +981,27 @@ def test_rope_kv_append_boundary_rows(dt):
     eq, es = oracle.quantize_int8(ko2.numpy().reshape(seq * 2, 128))
     assert_exact(kc.numpy().reshape(seq * 2, 128), eq, "k codes vs oracle")
     no_device_error()
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f32"])
+@pytest.mark.parametrize("rows, cols", [(1, 8193), (2, 20001), (16, 16384), (17, 16384), (3, 8192), (16, 8200)])
+def test_argmax_of_few_rows_spread_over_blocks(dt, rows, cols):
+    """Up to 16 rows of more than a segment are cut over blocks; ties across the cuts go to the
+    first, NaN at index 0 wins, and the slots are left zero for the next call and the flat argmax."""
+    rng = np.random.default_rng(rows * cols)
+    x = sample(rng, (rows, cols), dt)
+    top = f32_to_bf16(np.full(1, 9.0, np.float32))[0] if dt == "bf16" else np.float32(9.0)
+    for r in range(rows):
+        x[r, [cols // 3, cols - 1]] = top
+    if rows > 1:
+        x[1, 0] = 0x7FC0 if dt == "bf16" else np.nan
+    want_i, want_v = zip(*(oracle.argmax(x[r]) for r in range(rows)))
+    t = dev(x, DTS[dt])
+    for _ in range(2):
+        idx, val = empty((rows,), L.DataType.I64), empty((rows,), DTS[dt])
+        L.Ops.argmax_rows(idx, val, t)
+        assert_exact(idx.numpy(), np.array(want_i, np.int64))
+        assert_exact(val.numpy(), np.array(want_v, x.dtype))
+    fi, fv = empty((1,), L.DataType.I64), empty((1,), DTS[dt])
+    L.Ops.argmax(fi, fv, dev(x[:1], DTS[dt]))
+    assert fi.numpy()[0] == want_i[0]
