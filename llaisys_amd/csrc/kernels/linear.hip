@@ -45,14 +45,20 @@ struct LinearArgs {
     const float *scale;  // INT8 only
     const void *bias;    // T, or null
     int M, N, K;
+    bool swiglu; // (linearSkinny) w, scale and bias have 2 N rows, the gate's first
 };
 
 // Few rows (M <= 16, decode): HBM-bound on the weights; the skinny MFMA loop of
 // linear_common.hpp over one set of 16 channels, x rows >= M entering as zeros.  The waves'
-// 16 x 16 partials are summed in LDS in wave order.
-template <typename T, bool kInt8>
+// 16 x 16 partials are summed in LDS in wave order.  With kSw a block takes the 16 gate rows and the
+// 16 up rows of its channels and finishes with swiglu of the two, rounded to T as the separate
+// op would read them (each set sums as its own launch does: the same bits).  A launch costs about
+// 2.4 us beside its bytes: 5 rows, 1536 -> 2 x 8960, bf16, 2 x 6.9 us and a swiglu launch -> one launch; the layer of 5 tokens
+// 63.9 -> 59.0 us.
+template <typename T, bool kInt8, bool kSw>
 __global__ void __launch_bounds__(1024)
     linearSkinny(LinearArgs a) {
+    constexpr int R = kSw ? 2 : 1;
     // dynamic LDS, sized by the launch: nw transpose tiles, then nw partial tiles
     extern __shared__ __align__(16) char smem[];
     const int nw = int(blockDim.x) / kWave;
@@ -60,8 +66,8 @@ __global__ void __launch_bounds__(1024)
     const int lane = int(threadIdx.x) % kWave;
     const int r16 = lane % 16, g4 = lane / 16;
     const int n0 = int(blockIdx.x) * 16;
-    char *tile = smem + size_t(wave) * 16 * skinnyPitch(kInt8);
-    float(*red)[256] = reinterpret_cast<float(*)[256]>(smem + nw * 16 * skinnyPitch(kInt8));
+    char *tile = smem + size_t(wave) * R * 16 * skinnyPitch(kInt8);
+    float(*red)[R][256] = reinterpret_cast<float(*)[R][256]>(smem + nw * R * 16 * skinnyPitch(kInt8));
     const char *xrow = static_cast<const char *>(a.x) + size_t(min(r16, a.M - 1)) * a.K * 2;
     const bool xlane = r16 < a.M;
     const v4u z4 = {0u, 0u, 0u, 0u};
@@ -69,21 +75,34 @@ __global__ void __launch_bounds__(1024)
         const v4u v = *reinterpret_cast<const v4u *>(xrow + size_t(k < a.K ? k : 0) * 2);
         return xlane && k < a.K ? v : z4;
     };
-    f32x4 acc[1] = {{0.0f, 0.0f, 0.0f, 0.0f}};
-    const int rows0[1] = {n0};
-    skinnyGroups<T, kInt8, 1>(acc, static_cast<const char *>(a.w), rows0, a.N, a.K, tile, wave, nw, lane, xop);
+    f32x4 acc[R];
+    int rows0[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        acc[r] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        rows0[r] = n0 + r * a.N;
+    }
+    skinnyGroups<T, kInt8, R>(acc, static_cast<const char *>(a.w), rows0, R * a.N, a.K, tile, wave, nw, lane, xop);
     // D[m = 4 g + e][n = r16]
 #pragma unroll
-    for (int e = 0; e < 4; ++e) red[wave][(4 * g4 + e) * 16 + r16] = acc[0][e];
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) red[wave][r][(4 * g4 + e) * 16 + r16] = acc[r][e];
     __syncthreads();
     for (int t = int(threadIdx.x); t < 16 * a.M; t += int(blockDim.x)) {
         const int m = t / 16, n = n0 + t % 16;
         if (n < a.N) {
-            float s = 0.0f;
-            for (int w = 0; w < nw; ++w) s += red[w][t];
-            if constexpr (kInt8) s = a.scale[n] * s;
-            if (a.bias) s = s + Fmt<T>::get(a.bias, n);
-            Fmt<T>::put(a.out, size_t(m) * a.N + n, s);
+            float y[R];
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                float s = 0.0f;
+                for (int w = 0; w < nw; ++w) s += red[w][r][t];
+                if constexpr (kInt8) s = a.scale[n + r * a.N] * s;
+                if (a.bias) s = s + Fmt<T>::get(a.bias, n + r * a.N);
+                y[r] = s;
+            }
+            if constexpr (kSw) y[0] = SwigluOp::apply(Fmt<T>::round(y[0]), Fmt<T>::round(y[1]));
+            Fmt<T>::put(a.out, size_t(m) * a.N + n, y[0]);
         }
     }
 }
@@ -320,7 +339,10 @@ void launch(const LinearArgs &a, hipStream_t s) {
                 // per group of 128 k
                 const int tiles = (a.N + 15) / 16, nw = skinnyWaves(a.N, a.K);
                 const size_t lds = size_t(nw) * (16 * skinnyPitch(kInt8) + 256 * sizeof(float));
-                linearSkinny<T, kInt8><<<unsigned(tiles), unsigned(nw * kWave), lds, s>>>(a);
+                if (a.swiglu)
+                    linearSkinny<T, kInt8, true><<<unsigned(tiles), unsigned(nw * kWave), 2 * lds, s>>>(a);
+                else
+                    linearSkinny<T, kInt8, false><<<unsigned(tiles), unsigned(nw * kWave), lds, s>>>(a);
                 return;
             }
         }
@@ -350,13 +372,21 @@ void dispatch(const LinearArgs &a, llaisysDataType_t dt, hipStream_t s) {
 
 } // namespace
 
-bool linearSwigluFused(const LinearCall &c) { return gemmTakes(c); }
+// Rows 3 .. 16 of the 16-bit types: linearSkinny for one launch and for two alike (its waves' share
+// of K depends on N and K only), while the block's transpose tiles and partials fit LDS.
+bool linearSwigluFused(const LinearCall &c) {
+    const auto al = [](const void *p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+    if (gemmTakes(c)) return true;
+    if (c.dt == LLAISYS_DTYPE_F32 || c.rows <= 2 || c.rows > 16 || c.K == 0 || c.K % (c.scale ? 16 : 8) || !al(c.x) || !al(c.w))
+        return false;
+    return 2 * skinnyWaves(int(c.N), int(c.K)) * (16 * skinnyPitch(c.scale != nullptr) + 1024) <= 150 * 1024;
+}
 
 size_t linearWorkspaceBytes(const LinearCall &c) { return gemmTakes(c) ? gemmWorkspaceBytes(c) : 0; }
 
 void linear(const LinearCall &c, void *ws, size_t ws_bytes, hipStream_t s) {
     if (gemmTakes(c)) return gemm(c, ws, ws_bytes, s);
-    const LinearArgs a{c.out, c.x, c.w, c.scale, c.bias, int(c.rows), int(c.N), int(c.K)};
+    const LinearArgs a{c.out, c.x, c.w, c.scale, c.bias, int(c.rows), int(c.N), int(c.K), c.swiglu};
     if (c.scale)
         dispatch<true>(a, c.dt, s);
     else

@@ -60,7 +60,8 @@ def test_16_bit_tiles(shape, dt):
 
 
 @pytest.mark.parametrize("dt", ["bf16", "f16", "f32"])
-@pytest.mark.parametrize("rows, in_f, out_f", [(2, 64, 100), (17, 528, 90), (64, 2064, 33), (100, 1536, 131), (300, 528, 1000),
+@pytest.mark.parametrize("rows, in_f, out_f", [(2, 64, 100), (3, 1536, 2000), (16, 4112, 4100), (5, 272, 33),
+                                               (17, 528, 90), (64, 2064, 33), (100, 1536, 131), (300, 528, 1000),
                                                (1100, 144, 4500)])
 def test_swiglu_epilogue_equals_separate_ops(rows, in_f, out_f, dt):
     """rms_norm -> gate / up -> swiglu with the swiglu in the linear's epilogue (or in its split
