@@ -34,12 +34,19 @@ void fillSplits(Plan &p, const LinearCall &c, size_t blocks, size_t least) {
     setSplits(p, c, std::min({blocks / tiles, ceilDiv(c.K, p.ks) / least, cap}));
 }
 
-// f32: 64 weight rows, the fewest row tiles that hold the rows.  Bound by the f32 MFMA rate (154
-// TFLOP/s measured on a large product): one decoder layer of 128 tokens (hidden 1536, intermediate
-// 8960) 30.2 ms with one thread per output -> 0.223 ms, gate / up + swiglu 89.6 us, down 43.4 us.
+// f32: tiles of 64 weight rows x 32 or 64 rows, 64 k per stage shared by two (64 rows) or four waves
+// per tile quarter, split until every CU has a block.  Bound by the f32 MFMA rate (154 TFLOP/s on
+// a large product, 93 reached here at 128 rows): one decoder layer of 128 tokens (hidden 1536,
+// intermediate 8960) 30.2 ms with one thread per output -> 0.187 ms.  Against tiles of 128 rows, whose
+// blocks number 3.3 per CU at two together: gate / up + swiglu 97 -> 77 us, down 48 -> 39 us, 1536 ->
+// 1536 23 -> 13.4 us.
 Plan planF32(const LinearCall &c) {
-    Plan p{GemmTile::k64x64, 64, c.rows <= 32 ? 32 : c.rows <= 64 ? 64 : 128, 32, 1, 0};
-    fillSplits(p, c, 512, 4);
+    Plan p{GemmTile::k64x64, 64, c.rows <= 32 ? 32 : 64, 64, 1, 0};
+    fillSplits(p, c, kCUs, 3);
+    // unsplit with up to 8 blocks per CU: half as many weight rows per block, for a finer last round
+    // (128 rows, 1536 -> 2 x 8960: 2.2 blocks per CU 94 us, 4.4 of half the size 77 us)
+    const size_t tiles = ceilDiv(c.swiglu ? 2 * c.N : c.N, 64) * ceilDiv(c.rows, p.bx);
+    if (p.splits == 1 && tiles <= 8 * kCUs) p.bw = 32;
     return p;
 }
 
@@ -120,12 +127,14 @@ size_t planBytes(const Plan &p, const LinearCall &c) {
 
 template <bool kSw>
 void launchF32(const Plan &p, const GemmArgs &a, hipStream_t s) {
-    if (p.bx == 32)
-        launchTile<F32, false, kSw, 64, 32, 1, 1, 2, 32, 4>(a, s);
-    else if (p.bx == 64)
-        launchTile<F32, false, kSw, 64, 64, 1, 2, 2, 32, 3>(a, s);
+    if (p.bx == 32 && p.bw == 32)
+        launchTile<F32, false, kSw, 32, 32, 1, 1, 4, 64, 3>(a, s);
+    else if (p.bx == 32)
+        launchTile<F32, false, kSw, 64, 32, 2, 1, 4, 64, 2>(a, s);
+    else if (p.bw == 32)
+        launchTile<F32, false, kSw, 32, 64, 1, 2, 2, 64, 2>(a, s);
     else
-        launchTile<F32, false, kSw, 64, 128, 1, 4, 1, 32, 3>(a, s);
+        launchTile<F32, false, kSw, 64, 64, 2, 2, 2, 64, 2>(a, s);
     if (a.part) launchReduce<F32, false, kSw>(a, s);
 }
 
