@@ -445,11 +445,14 @@ __device__ __forceinline__ v4u codesToBf16(const v4u &raw, float sc) {
 // it fits, else its codes are converted on their way into LDS (the same operands, the same bits).
 // Keys past the cache read row 0 (finite wherever the reference's own output is; they weigh 0).
 //
-// What bounds it: a step is 24 MFMAs (768 cycles) and as much VALU work (16 exponentials per lane
-// and their two parts) per wave, two waves on a SIMD walking the same phases between barriers.
+// What bounds it: a step is 24 MFMAs (about 950 cycles) and 800 cycles of VALU work (16 exponentials
+// per lane and their two parts) per wave, two waves on a SIMD walking the same phases between barriers:
+// 1.9 us a step, near the sum of the phases.  Waves with tiles of their own and no barrier (two units
+// per wave), or four waves on a SIMD, came to the same 3.8 us per 256 keys, and running one unit half a
+// step behind the other spilled registers.
 // 2048 queries, 12 / 2 heads, bf16: 44.9 us with 16-query tiles and one wave per q head on 16 x 16
-// x 32 MFMAs (1 KB of LDS read per 16 MFMA cycles, CUs with early queries idle) -> 38.0 us; f16, 300
-// queries over 1500 INT8 keys: 479 us on the vector kernel -> 25.2 us.
+// x 32 MFMAs (1 KB of LDS read per 16 MFMA cycles, CUs with early queries idle) -> 34.9 us; f16, 300
+// queries over 1500 INT8 keys: 479 us on the vector kernel -> 23 us.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -516,6 +519,12 @@ __device__ __forceinline__ void visibleRange(size_t total, size_t seq, size_t q0
     least = q1 < wrapped ? total : visibleKeys(total, seq, q0 < wrapped ? wrapped : q0);
 }
 
+// The value of the lane 32 away
+__device__ __forceinline__ float otherHalf(float v) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(threadIdx.x & 32 ? r[0] : r[1]);
+}
+
 template <typename T, bool kInt8, int D, bool kHeads>
 __global__ void __launch_bounds__(kWave * 2 * kSplits, 2)
     attnPrefill(AttnArgs a) {
@@ -568,7 +577,14 @@ __global__ void __launch_bounds__(kWave * 2 * kSplits, 2)
         return v ? 4 * ((r >> 1) & 1) : (r >> 1) & 7;
     };
     // This wave's share of a step's loads: its split's K tile (unit 0) or V tile (unit 1).  Elements:
-    // load j fills 1 KB, rows j (1024 / RB) + lane / C.  Codes: lane l takes 16-code pieces l, l + 64, ...
+    // load j fills 1 KB, rows j kRows + lane / C: the row swizzles are those of lane / C, with bits 2 and 3 of
+    // the chunk flipped by j % 4 for K, so the lane offsets are formed once and the rest of an address is
+    // wave-uniform.  Codes: lane l takes 16-code pieces l, l + 64, ...
+    constexpr int kRows = 1024 / RB;
+    const uint32_t rowB = uint32_t(a.nkvh) * RB;
+    uint32_t off[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) off[j] = uint32_t(lane / C) * rowB + 16 * ((lane % C) ^ swzRow(unit, j * kRows + lane / C));
     const char *cache = static_cast<const char *>(unit ? a.v : a.k);
     const float *cscale = unit ? a.vs : a.ks;
     char *const mine = lds + split * 2 * kTileB + unit * kTileB;
@@ -588,12 +604,26 @@ __global__ void __launch_bounds__(kWave * 2 * kSplits, 2)
                 csc[j] = cscale[key];
             }
         } else {
+            const char *base = cache + (t0 * size_t(a.nkvh) + size_t(g)) * RB; // wave-uniform
+            // in scalar registers, formed anew each time: no per-load pointers are kept across the loop
+            const uint64_t bits = reinterpret_cast<uint64_t>(base);
+            base = reinterpret_cast<const char *>(uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(int(bits)))) |
+                                                  uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(int(bits >> 32)))) << 32);
+            char *dst = mine + stage * kStageB;
+            if (t0 + 32 <= a.total) {
 #pragma unroll
-            for (int j = 0; j < kLoads; ++j) {
-                const int row = j * (1024 / RB) + lane / C, chunk = (lane % C) ^ swzRow(unit, row);
-                const size_t key = (t0 + row < a.total ? t0 + row : 0) * size_t(a.nkvh) + size_t(g);
-                __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1))) *)(cache + key * RB + 16 * chunk),
-                                                 (void __attribute__((address_space(3))) *)(mine + stage * kStageB + j * 1024), 16, 0, 0);
+                for (int j = 0; j < kLoads; ++j)
+                    __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1))) *)(base + size_t(j * kRows) * rowB + off[j % 4]),
+                                                     (void __attribute__((address_space(3))) *)(dst + j * 1024), 16, 0, 0);
+            } else { // rows past the cache read row 0
+#pragma unroll
+                for (int j = 0; j < kLoads; ++j) {
+                    const bool in = t0 + size_t(j * kRows + lane / C) < a.total;
+                    const char *src = in ? base + size_t(j * kRows) * rowB + off[j % 4]
+                                         : cache + size_t(g) * RB + (off[j % 4] - uint32_t(lane / C) * rowB);
+                    __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1))) *)(src),
+                                                     (void __attribute__((address_space(3))) *)(dst + j * 1024), 16, 0, 0);
+                }
             }
         }
     };
@@ -613,10 +643,13 @@ __global__ void __launch_bounds__(kWave * 2 * kSplits, 2)
         }
     };
 
-    // this lane's K row (A row n) and V row pieces within a tile
+    // This lane's operand addresses within a tile: K row krow (A row n), the chunk of step st by XOR with
+    // 32 st; V pieces (4 columns of a row) of rows 8 h2 + (lane % 16) / 4, + 4 and + 16, the column tile dt
+    // by XOR with 64 dt.
     const int krow = 16 * (n / 16) + 8 * ((n >> 2) & 1) + 4 * ((n >> 3) & 1) + n % 4;
-    const int ksw = swzRow(false, krow);
-    const int vrow = 8 * h2 + (lane % 16) / 4; // and + 4, + 16
+    const int kaddr = krow * RB + 16 * (h2 ^ swzRow(false, krow));
+    const int vrow = 8 * h2 + (lane % 16) / 4;
+    const int vaddr = vrow * RB + 16 * ((2 * (lane / 16 % 2) + (lane % 4) / 2) ^ swzRow(true, vrow)) + 8 * (lane % 2);
     if (steps > 0) issue(0, 0);
     for (int it = 0; it < steps; ++it) {
         const int buf = it & 1;
@@ -631,16 +664,16 @@ __global__ void __launch_bounds__(kWave * 2 * kSplits, 2)
         for (int i = 0; i < 16; ++i) s[i] = 0.0f;
 #pragma unroll
         for (int st = 0; st < QS; ++st)
-            s = mfma32<T>(*reinterpret_cast<const v4u *>(kt + krow * RB + 16 * ((2 * st + h2) ^ ksw)), qreg[st], s);
+            s = mfma32<T>(*reinterpret_cast<const v4u *>(kt + (kaddr ^ (32 * st))), qreg[st], s);
         if (kt0 + 32 > least) { // the causal diagonal or the cache's end (block-uniform): mask
-            const int nvis = int(min(vis_q - min(vis_q, kt0), size_t(32)));
+            const int nvis = int(min(vis_q - min(vis_q, kt0), size_t(32))) - 8 * h2;
 #pragma unroll
-            for (int i = 0; i < 16; ++i) s[i] = 16 * (i / 8) + 8 * h2 + i % 8 < nvis ? s[i] : -INFINITY;
+            for (int i = 0; i < 16; ++i) s[i] = 16 * (i / 8) + i % 8 < nvis ? s[i] : -INFINITY;
         }
         float mx = m;
 #pragma unroll
         for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[i]);
-        mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
+        mx = fmaxf(mx, otherHalf(mx));
         // exp(scale (s - max)) as 2^(s c2 - max c2); a masked key (-inf) gets weight 0: mc = 0 while
         // every score is -inf keeps it 0 rather than NaN, with no per-score select
         const float mc = (mx == -INFINITY ? 0.0f : mx * c2) - kBias;
@@ -664,21 +697,21 @@ __global__ void __launch_bounds__(kWave * 2 * kSplits, 2)
 #pragma unroll
             for (int w = 0; w < 4; ++w) splitPair<T>(s[8 * kg + 2 * w], s[8 * kg + 2 * w + 1], hw[w], lw[w]);
             const v4u phi = {hw[0], hw[1], hw[2], hw[3]}, plo = {lw[0], lw[1], lw[2], lw[3]};
-            const int r0 = 16 * kg + vrow, r1 = r0 + 4;
-            const char *v0 = vt + r0 * RB + 8 * (lane % 2), *v1 = vt + r1 * RB + 8 * (lane % 2);
-            const int s0 = swzRow(true, r0), s1 = swzRow(true, r1);
+            v4u vv[DT];
 #pragma unroll
             for (int dt = 0; dt < DT; ++dt) {
-                // columns 32 dt + 16 (lane / 16 % 2) + 4 (lane % 4) ..: half lane % 2 of a chunk
-                const int ch = 4 * dt + 2 * (lane / 16 % 2) + (lane % 4) / 2;
-                const uint64_t e0 = ldsReadTr16(v0 + 16 * (ch ^ s0)), e1 = ldsReadTr16(v1 + 16 * (ch ^ s1));
-                const v4u vv = {uint32_t(e0), uint32_t(e0 >> 32), uint32_t(e1), uint32_t(e1 >> 32)};
-                o[dt] = mfma32<T>(vv, phi, o[dt]);
-                o[dt] = mfma32<T>(vv, plo, o[dt]);
+                const char *vp = vt + (vaddr ^ (64 * dt)) + 16 * kg * RB;
+                const uint64_t e0 = ldsReadTr16(vp), e1 = ldsReadTr16(vp + 4 * RB);
+                vv[dt] = v4u{uint32_t(e0), uint32_t(e0 >> 32), uint32_t(e1), uint32_t(e1 >> 32)};
             }
+            // (all column tiles before the second part: no MFMA waits for the one before it)
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) o[dt] = mfma32<T>(vv[dt], phi, o[dt]);
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) o[dt] = mfma32<T>(vv[dt], plo, o[dt]);
         }
     }
-    lsum += __shfl_xor(lsum, 32, kWave);
+    lsum += otherHalf(lsum);
 
     // merge the splits: every wave leaves (max, sum, output) in LDS, then wave (u, s) finishes the
     // column tiles s, s + kSplits, .. of unit u
