@@ -45,26 +45,29 @@ struct NormLinArgs {
 };
 
 
-template <typename T, bool kInt8, int G, int VMAX, bool kSwiglu, int U, int NW>
+// CH: output channels per wave
+template <typename T, bool kInt8, int G, int VMAX, bool kSwiglu, int U, int NW, int CH>
 __global__ void __launch_bounds__(NW * kWave)
     linearNormGemv(NormLinArgs a) {
     using F = Fmt<T>;
     constexpr int E = kInt8 ? 16 : 8;  // weight elements per 16-byte chunk
-    constexpr int R = kSwiglu ? 2 : 1; // weight rows per wave; U: chunks per lane and row per pass
+    // weight rows per wave: its channels' (gate) rows, then with swiglu their up rows; U: chunks per
+    // lane and row per pass
+    constexpr int R = (kSwiglu ? 2 : 1) * CH;
     static_assert(G == kWave || G == 256, "norm group: one wave or 4 waves");
     // a 4-wave norm group reduces through block-wide barriers, which every wave must reach
     static_assert(G == kWave || NW == 4, "a 256-lane norm group spans the whole block");
     extern __shared__ __align__(16) char xs[]; // the normalised row, K elements of T
     __shared__ float red[256 / kWave];
     const int lane = int(threadIdx.x) % kWave;
-    const int n = int(blockIdx.x) * NW + int(threadIdx.x) / kWave; // wave-uniform
-    const bool live = n < a.N; // a wave past the last channel loads a valid row, stores nothing
+    const int n0 = (int(blockIdx.x) * NW + int(threadIdx.x) / kWave) * CH; // wave-uniform
+    const bool live = n0 < a.N; // a wave past the last channel loads a valid row, stores nothing
     const int nc = a.K / E;    // K % E == 0
     const size_t rowB = size_t(a.K) * (kInt8 ? 1 : 2);
     const char *wrow[R];
 #pragma unroll
     for (int r = 0; r < R; ++r)
-        wrow[r] = static_cast<const char *>(a.w) + (size_t(live ? n : a.N - 1) + size_t(r) * a.N) * rowB;
+        wrow[r] = static_cast<const char *>(a.w) + (size_t(min(n0 + r % CH, a.N - 1)) + size_t(r / CH) * a.N) * rowB;
     // The first pass's weight chunks are requested before the norm, so that their latency
     // overlaps it (a chunk past the row end reads chunk 0 and is skipped below).
     v4u wv[R][U];
@@ -122,35 +125,48 @@ __global__ void __launch_bounds__(NW * kWave)
     float y[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-        const int ch = n + r * a.N;
+        const int ch = min(n0 + r % CH, a.N - 1) + r / CH * a.N;
         float s = waveGroupReduce<kWave, SumOp>(acc[r]);
         if constexpr (kInt8) s = a.scale[ch] * s;
         if (a.bias) s = s + F::get(a.bias, ch);
         y[r] = s;
     }
     if (lane == 0) {
-        if constexpr (kSwiglu)
-            F::put(a.out, n, SwigluOp::apply(F::round(y[0]), F::round(y[1])));
-        else
-            F::put(a.out, n, y[0]);
+#pragma unroll
+        for (int c = 0; c < CH; ++c) {
+            if (n0 + c >= a.N) break;
+            if constexpr (kSwiglu)
+                F::put(a.out, n0 + c, SwigluOp::apply(F::round(y[c]), F::round(y[CH + c])));
+            else
+                F::put(a.out, n0 + c, y[c]);
+        }
     }
 }
 
 // Waves per block: 8 for up to 4096 channels with a one-wave norm group (twice the channels
 // per norm; q/k/v [2048, 1536] 4.01 -> 3.68 us INT8, 4.66 -> 4.00 us bf16), else 4 (with 8:
 // gate/up + swiglu [2 x 8960, 1536] 9.99 -> 10.46 us INT8, 16 waves 12.67 us).
+// Channels per wave: 2 where one each would take more waves than the chip holds (256 CUs x 32), so that
+// no second round of blocks forms the row again and x is unpacked for twice the rows: INT8 [17920,
+// 1536] 11.83 -> 10.09 us, gate/up + swiglu [2 x 8960, 1536] 10.34 -> 9.97 us; bf16 [17920, 1536] 12.57 ->
+// 11.75 us.  16-bit gate/up rows keep one (11.93 -> 12.54 us with two), and 4 channels lose for INT8
+// gate/up (12.44 us).
+constexpr int kWavesAtOnce = 256 * 32;
+
 template <typename T, bool kInt8, bool kSwiglu, int U>
 void launchU(const NormLinArgs &a, const RowPlan &plan, hipStream_t s) {
     const size_t lds = size_t(a.K) * 2;
     const unsigned b4 = unsigned((a.N + 3) / 4);
     if (plan.group == kWave && a.N <= 4096)
-        linearNormGemv<T, kInt8, kWave, 4, kSwiglu, U, 8><<<unsigned((a.N + 7) / 8), 512, lds, s>>>(a);
+        linearNormGemv<T, kInt8, kWave, 4, kSwiglu, U, 8, 1><<<unsigned((a.N + 7) / 8), 512, lds, s>>>(a);
+    else if (plan.group == kWave && a.N > kWavesAtOnce && (kInt8 || !kSwiglu))
+        linearNormGemv<T, kInt8, kWave, 4, kSwiglu, U, 4, 2><<<unsigned((a.N + 7) / 8), 256, lds, s>>>(a);
     else if (plan.group == kWave)
-        linearNormGemv<T, kInt8, kWave, 4, kSwiglu, U, 4><<<b4, 256, lds, s>>>(a);
+        linearNormGemv<T, kInt8, kWave, 4, kSwiglu, U, 4, 1><<<b4, 256, lds, s>>>(a);
     else if (plan.vmax == 4)
-        linearNormGemv<T, kInt8, 256, 4, kSwiglu, U, 4><<<b4, 256, lds, s>>>(a);
+        linearNormGemv<T, kInt8, 256, 4, kSwiglu, U, 4, 1><<<b4, 256, lds, s>>>(a);
     else
-        linearNormGemv<T, kInt8, 256, 8, kSwiglu, U, 4><<<b4, 256, lds, s>>>(a);
+        linearNormGemv<T, kInt8, 256, 8, kSwiglu, U, 4, 1><<<b4, 256, lds, s>>>(a);
 }
 
 // Chunks per lane and pass: the whole row in one pass while it is at most 4 chunks per lane
