@@ -133,8 +133,9 @@ __C {
      * exceed the scratch -- queries x q heads x (head_dim + 2) x 4 KiB, e.g. more than 47
      * query-heads at head_dim 128 -- fails with a message.  A bf16 prefill (16 or more
      * queries, head_dim 128) dequantizes the caches into the scratch when they fit and
-     * otherwise converts the codes inside its kernel.  Calls on one GPU share the scratch:
-     * calls that overlap (other threads or streams) race. */
+     * otherwise converts the codes inside its kernel (its split partials take at most 8 MiB of
+     * it).  Calls on one GPU share the scratch: calls that overlap (other threads or streams)
+     * race. */
     __export void llaisysSelfAttentionInt8KVNoAlloc(llaisysTensor_t attn_val, llaisysTensor_t q,
                                                     llaisysTensor_t k_codes, llaisysTensor_t k_scale,
                                                     llaisysTensor_t v_codes, llaisysTensor_t v_scale,
@@ -164,7 +165,7 @@ __C {
      * llaisysLinearW8A16 when weight_scale is non-NULL; out = y, or with swiglu != 0 out[m][n] =
      * swiglu(gate = y[m][n], up = y[m][n + Nw/2]) for a weight of Nw rows (out [rows, Nw/2]).
      * bias NULL or zero-element means no bias.  One launch for one row; other row counts run
-     * the ops one after another. */
+     * the norm and then the linear, with swiglu in its epilogue or after it. */
     __export void llaisysRmsNormLinear(llaisysTensor_t out, llaisysTensor_t residual_out,
                                        llaisysTensor_t in, llaisysTensor_t residual,
                                        llaisysTensor_t norm_weight, float eps,

@@ -14,15 +14,15 @@
 // exp through the hardware exp2, and (sum p v) / (sum p) instead of sum (p / sum) v.  The
 // tests bound the difference by the f32 accumulation error of the reference itself.
 //
-// Design, three kernels (the launcher at the end picks one):
+// Design (the launcher at the end picks the kernel):
 //  - attnPrefill (bf16 / f16, head_dim 64 or 128, >= 16 queries): 32 queries of two q heads per
 //    block on v_mfma_f32_32x32x16, the keys split over the block's waves and, where the blocks
 //    leave CUs idle, over blocks (merged by attnCombineFew / attnCombine).
 //  - attnDecodeMfma (bf16 q, head_dim 128, fewer queries: decode, cache in bf16 or INT8):
 //    HBM-bound; the key range is cut into chunks, one block per (query, kv head, chunk) with
 //    the kv head's q heads as the MFMA columns; attnCombine merges the chunk partials.
-//  - attnGroup (f32, fewer queries in f16 or with head_dim 64): one wavefront per q head, the waves of a block
-//    being q heads of one kv head (they read the same K / V rows).  A key row of D elements
+//  - attnGroup (f32, fewer queries in f16 or with head_dim 64): one wavefront per q head, the
+//    waves of a block being q heads of one kv head (they read the same K / V rows).  A key row of D elements
 //    is spread over R = D / 8 lanes, 8 elements per lane, so one load instruction covers
 //    64 / R keys; per batch of U instructions the wave forms its scores (8 FMAs, a butterfly
 //    over R lanes), updates the running max once and folds p * v into per-lane

@@ -39,9 +39,8 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kXcds = 8; // accelerator complex dies, each with its own L2
 
-
 // A chunk of K past the row end is read from here: zeros add nothing to a sum.
-static __device__ const uint32_t kZeroChunk[4] = {0u, 0u, 0u, 0u};
+static __device__ const __align__(16) uint32_t kZeroChunk[4] = {0u, 0u, 0u, 0u};
 
 // Slot XOR of row r when a row is C chunks of 16 bytes: 16 consecutive rows reading one logical
 // chunk touch all 16 chunk positions of 256 bytes of LDS.
