@@ -154,9 +154,14 @@ __global__ void __launch_bounds__(NWW *NWX *NWK * 64)
         }
     }
     const bool tail = a.K % KS != 0 && kt0 + nk == nk_all; // the last stage reaches past the rows
-    const auto issue = [&](int kt) { // called for kt = 0, 1, ..: the sources move on with it
+    // Called for kt = 0, 1, ..: the sources move on with it.  `steady`, here and in the stages below,
+    // is a compile-time promise that kt is not the last stage: the loop over all but the last S
+    // stages then has no branch around its loads and one constant wait, and the compiler places the
+    // loads among the LDS reads and MFMAs (2048 rows of gate / up / swiglu 129.8 -> 127.1 us, one
+    // [8960, 1536] 83.2 -> 79.4 in tiles of 192 x 256, 79.8 -> 79.0 in 192 x 128; 96 x 128 -8%).
+    const auto issue = [&](int kt, auto steady) {
         char *dst = lds + (kt % S) * kStageB;
-        if (__builtin_expect(tail && kt == nk - 1, 0)) {
+        if (!steady && tail && kt == nk - 1) {
 #pragma unroll
             for (int i = 0; i < kLoads; ++i) {
                 const int q = slot(i);
@@ -187,7 +192,7 @@ __global__ void __launch_bounds__(NWW *NWX *NWK * 64)
     const int wbase = (ww0 + r32) * WB, xbase = BW * WB + (wx0 + r32) * XB;
 #pragma unroll
     for (int st = 0; st < S - 1; ++st)
-        if (st < nk) issue(st);
+        if (st < nk) issue(st, std::false_type{});
     if constexpr (kPipe) {
         // One wave per SIMD: the operands of a pair of steps (one 16-code chunk per weight row) are
         // read from LDS while the MFMAs of the pair before run, also across stages, so a stage is
@@ -220,13 +225,13 @@ __global__ void __launch_bounds__(NWW *NWX *NWK * 64)
                     for (int j = 0; j < TX; ++j) acc[i][j] = mfmaChunk<T>(fa, o.x[j][c], acc[i][j]);
                 }
         };
-        const auto stage = [&](int kt, Ops &cur, Ops &nxt) {
-            if (kt + S - 2 < nk) // stage kt + 1 has landed
+        const auto stage = [&](int kt, Ops &cur, Ops &nxt, auto steady) {
+            if (steady || kt + S - 2 < nk) // stage kt + 1 has landed
                 waitVmcnt<kLoads * (S - 3)>();
             else
                 waitVmcnt<0>();
             stageBarrier(); // for every wave; stage kt - 1 is no longer read
-            if (kt + S - 1 < nk) issue(kt + S - 1);
+            if (steady || kt + S - 1 < nk) issue(kt + S - 1, steady);
 #pragma unroll
             for (int p = 0; p < kPairs; ++p) {
                 Ops &c = p % 2 ? nxt : cur, &n = p % 2 ? cur : nxt;
@@ -252,65 +257,76 @@ __global__ void __launch_bounds__(NWW *NWX *NWK * 64)
         ldsBarrier();
         fetch(o0, 0, 0);
         if constexpr (kPairs % 2 == 0) {
-            for (int kt = 0; kt < nk; ++kt) stage(kt, o0, o1);
+            int kt = 0;
+            for (; kt + S < nk; ++kt) stage(kt, o0, o1, std::true_type{});
+            for (; kt < nk; ++kt) stage(kt, o0, o1, std::false_type{});
         } else {
-            for (int kt = 0; kt < nk; kt += 2) {
-                stage(kt, o0, o1);
-                if (kt + 1 < nk) stage(kt + 1, o1, o0);
+            int kt = 0;
+            for (; kt + 1 + S < nk; kt += 2) {
+                stage(kt, o0, o1, std::true_type{});
+                stage(kt + 1, o1, o0, std::true_type{});
+            }
+            for (; kt < nk; kt += 2) {
+                stage(kt, o0, o1, std::false_type{});
+                if (kt + 1 < nk) stage(kt + 1, o1, o0, std::false_type{});
             }
         }
-    } else
-    for (int kt = 0; kt < nk; ++kt) {
-        // this wave's loads of stage kt have landed (the stages after it may be in flight)
-        if (kt + S - 2 < nk)
-            waitVmcnt<kLoads * (S - 2)>();
-        else
-            waitVmcnt<0>();
-        ldsBarrier(); // every wave's have; stage kt - 1 is no longer read
-        if (kt + S - 1 < nk) issue(kt + S - 1);
-        const char *tile = lds + (kt % S) * kStageB;
-        // k order of a stage: 16-bit types, step st and half h: chunk 4 (st / 2) + 2 h + st % 2, so
-        // that the 16 codes of an INT8 chunk serve two steps; f32: chunk 2 st + h
-        constexpr int kSteps = XC / 2;
-        static_assert(kSteps % NWK == 0 && (kE == 4 || kSteps / 2 % NWK == 0), "the waves of a tile share its steps evenly");
-        if constexpr (kInt8) {
+    } else {
+        const auto stage = [&](int kt, auto steady) {
+            // this wave's loads of stage kt have landed (the stages after it may be in flight)
+            if (steady || kt + S - 2 < nk)
+                waitVmcnt<kLoads * (S - 2)>();
+            else
+                waitVmcnt<0>();
+            ldsBarrier(); // every wave's have; stage kt - 1 is no longer read
+            if (steady || kt + S - 1 < nk) issue(kt + S - 1, steady);
+            const char *tile = lds + (kt % S) * kStageB;
+            // k order of a stage: 16-bit types, step st and half h: chunk 4 (st / 2) + 2 h + st % 2, so
+            // that the 16 codes of an INT8 chunk serve two steps; f32: chunk 2 st + h
+            constexpr int kSteps = XC / 2;
+            static_assert(kSteps % NWK == 0 && (kE == 4 || kSteps / 2 % NWK == 0), "the waves of a tile share its steps evenly");
+            if constexpr (kInt8) {
 #pragma unroll
-            for (int pw = 0; pw < kSteps / 2 / NWK; ++pw) {
-                const int p = wk * (kSteps / 2 / NWK) + pw;
-                v4u ca[TW];
+                for (int pw = 0; pw < kSteps / 2 / NWK; ++pw) {
+                    const int p = wk * (kSteps / 2 / NWK) + pw;
+                    v4u ca[TW];
 #pragma unroll
-                for (int i = 0; i < TW; ++i)
-                    ca[i] = *reinterpret_cast<const v4u *>(tile + wbase + 32 * i * WB + 16 * ((2 * p + h2) ^ wsz));
+                    for (int i = 0; i < TW; ++i)
+                        ca[i] = *reinterpret_cast<const v4u *>(tile + wbase + 32 * i * WB + 16 * ((2 * p + h2) ^ wsz));
 #pragma unroll
-                for (int s2 = 0; s2 < 2; ++s2) {
-                    v4u fb[TX];
+                    for (int s2 = 0; s2 < 2; ++s2) {
+                        v4u fb[TX];
 #pragma unroll
-                    for (int j = 0; j < TX; ++j)
-                        fb[j] = *reinterpret_cast<const v4u *>(tile + xbase + 32 * j * XB + 16 * ((4 * p + 2 * h2 + s2) ^ xsz));
+                        for (int j = 0; j < TX; ++j)
+                            fb[j] = *reinterpret_cast<const v4u *>(tile + xbase + 32 * j * XB + 16 * ((4 * p + 2 * h2 + s2) ^ xsz));
 #pragma unroll
-                    for (int i = 0; i < TW; ++i) {
-                        const v4u fa = codesToT<T>(s2 ? v2u{ca[i].z, ca[i].w} : v2u{ca[i].x, ca[i].y});
+                        for (int i = 0; i < TW; ++i) {
+                            const v4u fa = codesToT<T>(s2 ? v2u{ca[i].z, ca[i].w} : v2u{ca[i].x, ca[i].y});
 #pragma unroll
-                        for (int j = 0; j < TX; ++j) acc[i][j] = mfmaChunk<T>(fa, fb[j], acc[i][j]);
+                            for (int j = 0; j < TX; ++j) acc[i][j] = mfmaChunk<T>(fa, fb[j], acc[i][j]);
+                        }
                     }
                 }
+            } else {
+#pragma unroll
+                for (int sw = 0; sw < kSteps / NWK; ++sw) {
+                    const int st = wk * (kSteps / NWK) + sw;
+                    const int c = kE == 2 ? 4 * (st / 2) + 2 * h2 + st % 2 : 2 * st + h2;
+                    v4u fa[TW], fb[TX];
+#pragma unroll
+                    for (int i = 0; i < TW; ++i) fa[i] = *reinterpret_cast<const v4u *>(tile + wbase + 32 * i * WB + 16 * (c ^ wsz));
+#pragma unroll
+                    for (int j = 0; j < TX; ++j) fb[j] = *reinterpret_cast<const v4u *>(tile + xbase + 32 * j * XB + 16 * (c ^ xsz));
+#pragma unroll
+                    for (int i = 0; i < TW; ++i)
+#pragma unroll
+                        for (int j = 0; j < TX; ++j) acc[i][j] = mfmaChunk<T>(fa[i], fb[j], acc[i][j]);
+                }
             }
-        } else {
-#pragma unroll
-            for (int sw = 0; sw < kSteps / NWK; ++sw) {
-                const int st = wk * (kSteps / NWK) + sw;
-                const int c = kE == 2 ? 4 * (st / 2) + 2 * h2 + st % 2 : 2 * st + h2;
-                v4u fa[TW], fb[TX];
-#pragma unroll
-                for (int i = 0; i < TW; ++i) fa[i] = *reinterpret_cast<const v4u *>(tile + wbase + 32 * i * WB + 16 * (c ^ wsz));
-#pragma unroll
-                for (int j = 0; j < TX; ++j) fb[j] = *reinterpret_cast<const v4u *>(tile + xbase + 32 * j * XB + 16 * (c ^ xsz));
-#pragma unroll
-                for (int i = 0; i < TW; ++i)
-#pragma unroll
-                    for (int j = 0; j < TX; ++j) acc[i][j] = mfmaChunk<T>(fa[i], fb[j], acc[i][j]);
-            }
-        }
+        };
+        int kt = 0;
+        for (; kt + S < nk; ++kt) stage(kt, std::true_type{});
+        for (; kt < nk; ++kt) stage(kt, std::false_type{});
     }
     if constexpr (NWK > 1) { // the waves' shares of a tile, added in wave order
         constexpr int kAcc = TW * TX * 16;
