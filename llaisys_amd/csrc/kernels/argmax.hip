@@ -196,7 +196,8 @@ __global__ void __launch_bounds__(kBlock)
 // index, makes a larger key; a block with no candidate (all -inf / NaN) skips it.  The
 // atomic returns its old value, and the wait for it orders the maximum before the block's
 // arrival count; the last block to arrive reads the key (and element 0) with device-scope
-// loads, finishes, and leaves key and counter zero.  Device-scope atomics are performed at
+// loads, finishes, and leaves key and counter zero.  -0 and +0 are equal, so they share a key
+// and the lower index wins between them; the sign of a zero winner is read back from its element.  Device-scope atomics are performed at
 // the device's coherence point, so no L2 write-back fence is needed between blocks.
 struct FlatSlots {
     unsigned counter; // the launch's arrival count (offset 0 of the scratch)
@@ -204,9 +205,10 @@ struct FlatSlots {
     unsigned long long key;
 };
 
+constexpr uint32_t kZeroOrder = 0x80000000u; // order bits of both zeros
 __device__ __forceinline__ uint32_t orderBits(float v) {
     const uint32_t b = __float_as_uint(v);
-    return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
+    return b > 0x80000000u ? ~b : (b | 0x80000000u);
 }
 
 // One vector of n elements per blockIdx.y, its slots at sl[blockIdx.y] and its results at that index.
@@ -241,6 +243,7 @@ __global__ void __launch_bounds__(kBlock)
         const uint32_t ob = uint32_t(key >> 32);
         m.v = __uint_as_float((ob & 0x80000000u) ? (ob & 0x7FFFFFFFu) : ~ob);
         m.i = int64_t(~uint32_t(key));
+        if (ob == kZeroOrder) m.v = Fmt<T>::get(vals, size_t(m.i));
     }
     finish<T>(m, x0_all, idx, i64, val, row);
     __hip_atomic_store(&sl->key, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

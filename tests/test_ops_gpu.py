@@ -1005,3 +1005,23 @@ def test_argmax_of_few_rows_spread_over_blocks(dt, rows, cols):
     fi, fv = empty((1,), L.DataType.I64), empty((1,), DTS[dt])
     L.Ops.argmax(fi, fv, dev(x[:1], DTS[dt]))
     assert fi.numpy()[0] == want_i[0]
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16", "f32"])
+@pytest.mark.parametrize("rows", [1, 2, 16, 17])
+@pytest.mark.parametrize("signs", [(-0.0, 0.0), (0.0, -0.0)])
+def test_argmax_zero_maximum_takes_the_first_sign(dt, rows, signs):
+    """-0 and +0 are equal: where the maximum is zero, the first of them wins, with its own sign, also
+    when the two lie in different blocks' segments (rows cut over blocks, a block per row, flat)."""
+    cols = 20001
+    x = np.full((rows, cols), -1.0, np.float32)
+    x[:, 5], x[:, cols - 3] = signs
+    x = {"bf16": lambda a: f32_to_bf16(a), "f16": lambda a: a.astype(np.float16), "f32": lambda a: a}[dt](x)
+    want_i, want_v = oracle.argmax_rows(x)
+    idx, val = empty((rows,), L.DataType.I64), empty((rows,), DTS[dt])
+    L.Ops.argmax_rows(idx, val, dev(x, DTS[dt]))
+    assert_exact(idx.numpy(), want_i)
+    assert_exact(val.numpy(), want_v)
+    fi, fv = empty((1,), L.DataType.I64), empty((1,), DTS[dt])
+    L.Ops.argmax(fi, fv, dev(x[0], DTS[dt]))
+    assert (fi.numpy()[0], fv.numpy().tobytes()) == (want_i[0], want_v[:1].tobytes())
