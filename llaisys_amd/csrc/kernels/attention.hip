@@ -443,7 +443,8 @@ __device__ __forceinline__ v4u codesToBf16(const v4u &raw, float sc) {
 // 16-byte chunks of a row are XOR-swizzled: K so that 16 rows' reads of one chunk touch all banks,
 // V so that the 64-byte pieces of 4 rows do.  An INT8 cache is dequantized into the workspace when
 // it fits, else its codes are converted on their way into LDS (the same operands, the same bits).
-// Keys past the cache read row 0 (finite wherever the reference's own output is; they weigh 0).
+// Keys past the cache read row 0 and weigh 0, as masked keys do; what a non-finite V element of
+// such a row leaves in the sums is replaced at the end (visibleSum).
 //
 // What bounds it: a step is 24 MFMAs (about 950 cycles) and 800 cycles of VALU work (16 exponentials
 // per lane and their two parts) per wave, two waves on a SIMD walking the same phases between barriers:
@@ -523,6 +524,42 @@ __device__ __forceinline__ void visibleRange(size_t total, size_t seq, size_t q0
 __device__ __forceinline__ float otherHalf(float v) {
     const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     return __uint_as_float(threadIdx.x & 32 ? r[0] : r[1]);
+}
+
+// Column col of sum p V over the keys [k0, end) of kv head g for one q row, p = 2^(dot c2 - mc):
+// a wave's work, 64 keys' weights at a time, only those keys' rows read.
+template <typename T, bool kInt8, int D>
+__device__ __forceinline__ float visibleSum(const AttnArgs &a, const uint16_t *qrow, int g, int col, size_t k0,
+                                            size_t end, float c2, float mc) {
+    using IO = RowIO<T, kInt8>;
+    using QO = RowIO<T, false>;
+    const int lane = int(threadIdx.x) % kWave;
+    float acc = 0.0f;
+    for (size_t kb = k0; kb < end; kb += kWave) {
+        const size_t krow = min(kb + size_t(lane), end - 1) * size_t(a.nkvh) + size_t(g);
+        float dot = 0.0f;
+#pragma unroll 1
+        for (int c = 0; c < D; c += 8) {
+            float qf[8], kf[8];
+            QO::unpack(QO::load(qrow, 0, D, c), 0.0f, qf);
+            IO::unpack(IO::load(a.k, krow, D, c), kInt8 ? a.ks[krow] : 0.0f, kf);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) dot = __builtin_fmaf(qf[e], kf[e], dot);
+        }
+        const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(dot, c2, -mc));
+        const int keys = int(min(end - kb, size_t(kWave)));
+#pragma unroll 1
+        for (int j = 0; j < keys; ++j) {
+            const size_t vrow = (kb + size_t(j)) * size_t(a.nkvh) + size_t(g);
+            float v;
+            if constexpr (kInt8)
+                v = Fmt<T>::round(float(static_cast<const int8_t *>(a.v)[vrow * D + col]) * a.vs[vrow]);
+            else
+                v = Fmt<T>::get(a.v, vrow * D + col);
+            acc = __builtin_fmaf(__shfl(p, j, kWave), v, acc);
+        }
+    }
+    return acc;
 }
 
 template <typename T, bool kInt8, int D, bool kHeads>
@@ -729,7 +766,7 @@ __global__ void __launch_bounds__(kWave * 2 * kSplits, 2)
             *reinterpret_cast<f32x4 *>(xo + ((((unit * kSplits + split) * DT + dt) * 4 + q) * kWave + lane) * 4) =
                 f32x4{o[dt][4 * q], o[dt][4 * q + 1], o[dt][4 * q + 2], o[dt][4 * q + 3]};
     ldsBarrier();
-    if (q0 + size_t(n) >= a.seq) return;
+    const bool live = q0 + size_t(n) < a.seq;
     float M = -INFINITY, L = 0.0f, f[kSplits];
 #pragma unroll
     for (int k = 0; k < kSplits; ++k) M = fmaxf(M, ml[unit][k][0][n]);
@@ -741,28 +778,58 @@ __global__ void __launch_bounds__(kWave * 2 * kSplits, 2)
     }
     const size_t ih = qi * a.nh + size_t(h);
     float *const part = a.nchunks > 1 ? a.part + (ih * size_t(a.nchunks) + c) * (D + 2) : nullptr;
-    const float inv = L > 0.0f ? 1.0f / L : 0.0f;
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) {
-        if (dt % kSplits != split) continue;
+    static_assert(DT <= kSplits, "a wave finishes one column tile at most");
+    if (split < DT) {
+        const int dt = split;
+        f32x4 O[4];
+        float z = 0.0f; // NaN where an output is not finite
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            f32x4 O = {0.0f, 0.0f, 0.0f, 0.0f};
+            O[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
             for (int k = 0; k < kSplits; ++k)
-                O += f[k] * *reinterpret_cast<const f32x4 *>(xo + ((((unit * kSplits + k) * DT + dt) * 4 + q) * kWave + lane) * 4);
+                O[q] += f[k] * *reinterpret_cast<const f32x4 *>(xo + ((((unit * kSplits + k) * DT + dt) * 4 + q) * kWave + lane) * 4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) z = __builtin_fmaf(O[q][e], 0.0f, z);
+        }
+        // The MFMA also multiplies V rows that a query does not see (past the diagonal, and the filler past
+        // the cache) by 0, and a visible infinity by a low part that may be 0 or negative: where an output is
+        // not finite though the weights are (L), the query's 32 columns are summed again over its own keys.
+        uint64_t redo = __ballot(live && z != z && L == L);
+        if (__builtin_expect(redo != 0, 0)) {
+            const float mc = (M == -INFINITY ? 0.0f : M * c2) - kBias;
+            uint32_t rows = uint32_t(redo) | uint32_t(redo >> 32);
+            while (rows) {
+                const int r = __builtin_ctz(rows);
+                rows &= rows - 1;
+                const size_t i = q0 + size_t(r);
+                const float y = visibleSum<T, kInt8, D>(a, static_cast<const uint16_t *>(a.q) + (i * a.nh + h) * D, g, 32 * dt + n, k0,
+                                                        min(k1, visibleKeys(a.total, a.seq, i)), c2, __shfl(mc, r, kWave));
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float ye = __shfl(y, 8 * q + 4 * h2 + e, kWave);
+                        O[q][e] = n == r ? ye : O[q][e];
+                    }
+            }
+        }
+        const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            if (!live) break;
             const int col = 32 * dt + 8 * q + 4 * h2;
             if (part) {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) part[col + e] = O[e];
+                for (int e = 0; e < 4; ++e) part[col + e] = O[q][e];
             } else {
                 using Cv = std::conditional_t<std::is_same_v<T, BF16>, Bf16Cvt, F16Cvt>; // the reference rounding
                 *reinterpret_cast<v2u *>(static_cast<uint16_t *>(a.out) + ih * D + col) =
-                    v2u{Cv::narrow(O[0] * inv) | (Cv::narrow(O[1] * inv) << 16), Cv::narrow(O[2] * inv) | (Cv::narrow(O[3] * inv) << 16)};
+                    v2u{Cv::narrow(O[q][0] * inv) | (Cv::narrow(O[q][1] * inv) << 16), Cv::narrow(O[q][2] * inv) | (Cv::narrow(O[q][3] * inv) << 16)};
             }
         }
     }
-    if (part && split == 0 && h2 == 0) {
+    if (part && live && split == 0 && h2 == 0) {
         part[D] = M * a.scale; // the scaled units attnCombine works in
         part[D + 1] = L;
     }

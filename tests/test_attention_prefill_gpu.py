@@ -7,6 +7,7 @@ import pytest
 
 import llaisys_amd as L
 import oracle
+from numerics import _as_f32 as as_f32
 from numerics import assert_attention_close, assert_exact
 from test_attention_gpu import AMD, DTS, attend, dev, sample
 
@@ -69,3 +70,54 @@ def test_no_alloc_prefill_over_a_split_cache():
     L.Ops.self_attention_int8kv(ref, tq, *t8, 0.0883883)
     L.Ops.self_attention_int8kv_noalloc(out, tq, *t8, 0.0883883)
     assert_exact(out.numpy(), ref.numpy(), "no alloc")
+
+
+def _bits(x, dt):
+    """f32 values (infinities and NaN among them) in the storage type."""
+    x = np.float32(x)
+    return {"bf16": lambda: np.uint16(x.view(np.uint32) >> 16), "f16": lambda: np.float16(x)}[dt]()
+
+
+def visible_attention(q, k, v, scale):
+    """The oracle over each query's own keys alone."""
+    seq, total = q.shape[0], k.shape[0]
+    rows = [oracle.self_attention(q[i:i + 1], k[:total - seq + i + 1], v[:total - seq + i + 1], scale) for i in range(seq)]
+    return np.concatenate(rows)
+
+
+# seq, total, nh, nkvh: the diagonal within one step, rows past the cache in a part-filled tile, an odd
+# group's two query blocks, and keys split over blocks
+NON_FINITE = [(40, 40, 4, 2), (33, 201, 3, 1), (40, 1100, 2, 1)]
+
+
+@pytest.mark.parametrize("int8", [False, True], ids=["plain", "int8"])
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("shape", NON_FINITE, ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan])
+def test_non_finite_v_reaches_only_queries_that_see_it(value, shape, dt, d, int8):
+    """An infinite or NaN V element of a later token leaves earlier queries as they were (the tiles hold
+    keys that a query does not see), and an infinite one that is seen gives an infinity, not NaN."""
+    seq, total, nh, nkvh = shape
+    rng = np.random.default_rng(zlib.crc32(repr((shape, dt, d)).encode()))
+    q, k, v = sample(rng, (seq, nh, d), dt), sample(rng, (total, nkvh, d), dt), sample(rng, (total, nkvh, d), dt)
+    scale = float(np.float32(1.0 / np.sqrt(d)))
+    late = total - seq // 2  # seen by the second half of the queries
+    if int8:
+        (kq, ks), (vq, vs) = oracle.quantize_int8(k), oracle.quantize_int8(v)
+        vs[late, 0] = value  # the whole row, zero codes NaN
+        k, v = (oracle.dequantize_int8(c, s, q.dtype) for c, s in ((kq, ks), (vq, vs)))
+    else:
+        v[late, 0, [3, d - 1]] = _bits(value, dt)
+        v[0, nkvh - 1, 17] = _bits(value, dt)  # what rows past the cache are read from
+    want = visible_attention(q, k, v, scale)
+    tq, out = dev(q, DTS[dt]), L.Tensor((seq, nh, d), DTS[dt], **AMD)
+    if int8:
+        L.Ops.self_attention_int8kv(out, tq, *(dev(a) for a in (kq, ks, vq, vs)), scale)
+        got = out.numpy()
+    else:
+        got = attend(q, k, v, scale, dt)
+    finite = np.where(np.isfinite(as_f32(v)), v, np.zeros_like(v))  # for the tolerance's max |v|
+    assert_attention_close(got, want, finite, f"{dt} {shape} d{d}")
+    got, want = as_f32(got), as_f32(want)
+    assert_exact(np.where(np.isinf(got), got, 0), np.where(np.isinf(want), want, 0), "infinities")
