@@ -271,7 +271,7 @@ __global__ void __launch_bounds__(kWave * kWaves)
         const size_t ih = i * a.nh + size_t(h0 + j);
         if (a.nchunks == 1) {
             // put: the reference rounding, also for a NaN carrying the caller's scale payload
-            Fmt<T>::put(a.out, ih * D + e, L > 0.0f ? O / L : 0.0f);
+            Fmt<T>::put(a.out, ih * D + e, L == 0.0f ? 0.0f : O / L);
         } else {
             float *pp = a.part + (ih * size_t(a.nchunks) + c) * (D + 2);
             pp[e] = O;
@@ -336,7 +336,7 @@ __global__ void __launch_bounds__(kCombineThreads)
     if (t < kCombineCols) {
         float O = 0.0f;
         for (int g = 0; g < kGroups; ++g) O += red[g * kCombineCols + t];
-        Fmt<T>::put(out, ih * D + col0 + t, L > 0.0f ? O / L : 0.0f);
+        Fmt<T>::put(out, ih * D + col0 + t, L == 0.0f ? 0.0f : O / L);
     }
 }
 
@@ -814,7 +814,7 @@ __global__ void __launch_bounds__(kWave * 2 * kSplits, 2)
                     }
             }
         }
-        const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+        const float inv = L == 0.0f ? 0.0f : 1.0f / L;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             if (!live) break;
@@ -856,7 +856,7 @@ __global__ void __launch_bounds__(256)
         for (int e = 0; e < 4; ++e) O[e] += pc[col + e] * f;
     }
 #pragma unroll
-    for (int e = 0; e < 4; ++e) Fmt<T>::put(out, ih * D + col + e, L > 0.0f ? O[e] / L : 0.0f);
+    for (int e = 0; e < 4; ++e) Fmt<T>::put(out, ih * D + col + e, L == 0.0f ? 0.0f : O[e] / L);
 }
 
 // ---- decode on MFMA (bf16 q / out, head_dim 128, cache in bf16 or INT8) ---------------
@@ -1068,7 +1068,7 @@ __global__ void __launch_bounds__(kWave * NW)
         }
         const size_t ih = i * a.nh + size_t(g * a.group + j);
         if (a.nchunks == 1) {
-            Fmt<BF16>::put(a.out, ih * D + e, L > 0.0f ? O / L : 0.0f);
+            Fmt<BF16>::put(a.out, ih * D + e, L == 0.0f ? 0.0f : O / L);
         } else {
             float *pp = a.part + (ih * size_t(a.nchunks) + c) * (D + 2);
             pp[e] = O;

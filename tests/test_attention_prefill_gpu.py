@@ -75,7 +75,7 @@ def test_no_alloc_prefill_over_a_split_cache():
 def _bits(x, dt):
     """f32 values (infinities and NaN among them) in the storage type."""
     x = np.float32(x)
-    return {"bf16": lambda: np.uint16(x.view(np.uint32) >> 16), "f16": lambda: np.float16(x)}[dt]()
+    return {"bf16": lambda: np.uint16(x.view(np.uint32) >> 16), "f16": lambda: np.float16(x), "f32": lambda: x}[dt]()
 
 
 def visible_attention(q, k, v, scale):
@@ -121,3 +121,23 @@ def test_non_finite_v_reaches_only_queries_that_see_it(value, shape, dt, d, int8
     assert_attention_close(got, want, finite, f"{dt} {shape} d{d}")
     got, want = as_f32(got), as_f32(want)
     assert_exact(np.where(np.isinf(got), got, 0), np.where(np.isinf(want), want, 0), "infinities")
+
+
+# seq, total, nh, nkvh, d: prefill in one piece and with the keys split over few and many blocks, decode
+# in one piece and split, head_dim 64
+BAD_SCORES = [(40, 40, 4, 2, 128), (33, 1100, 3, 1, 64), (16, 9000, 2, 1, 128), (5, 40, 4, 2, 128), (2, 3000, 12, 2, 128),
+              (3, 700, 4, 2, 64)]
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16", "f32"])
+@pytest.mark.parametrize("shape", BAD_SCORES, ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("value", [np.inf, np.nan])
+def test_non_finite_k_gives_nan_where_the_reference_does(value, shape, dt):
+    """A NaN or +Inf score makes its query's output NaN (not 0), a -Inf score weighs nothing, and
+    queries before the key are as they were, whether or not the keys are split over blocks."""
+    seq, total, nh, nkvh, d = shape
+    rng = np.random.default_rng(zlib.crc32(repr((shape, dt)).encode()))
+    q, k, v = sample(rng, (seq, nh, d), dt), sample(rng, (total, nkvh, d), dt), sample(rng, (total, nkvh, d), dt)
+    k[total - (seq + 1) // 2, 0, 9] = _bits(value, dt)
+    scale = 1.0 / np.sqrt(d)
+    assert_attention_close(attend(q, k, v, scale, dt), visible_attention(q, k, v, scale), v, f"{dt} {shape}")
