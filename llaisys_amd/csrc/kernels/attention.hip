@@ -1127,6 +1127,8 @@ constexpr size_t kPrefillPartBytes = size_t(8) << 20;
 bool planPrefill(Prefill &p, const AttnArgs &a, int d, int dv, bool int8, llaisysDataType_t dt) {
     if ((dt != LLAISYS_DTYPE_BF16 && dt != LLAISYS_DTYPE_F16) || !vecShape(a, d, dv, int8)) return false;
     if (a.total == 0 || a.seq < size_t(kMfmaQ) || !(a.scale > 0.0f) || !std::isfinite(a.scale)) return false;
+    // the kernel's lane offsets within one 1 KB load (512 / d key rows) have 32 bits
+    if (size_t(a.nkvh) * 1024 >= size_t(1) << 32) return false;
     p.heads = a.group % 2 == 0;
     p.slices = p.heads ? a.group / 2 : a.group;
     const size_t qb = (a.seq + (p.heads ? 31 : 63)) / (p.heads ? 32 : 64);
@@ -1142,6 +1144,19 @@ bool planPrefill(Prefill &p, const AttnArgs &a, int d, int dv, bool int8, llaisy
     p.part_bytes = n > 1 ? a.seq * size_t(a.nh) * n * size_t(d + 2) * sizeof(float) : 0;
     p.blocks *= n;
     return p.blocks < (size_t(1) << 31);
+}
+
+// Chunks of the vector kernel's keys.  A block's waves each take one step of keys per chunk when the
+// launch is split: about 2048 waves for decode, partials within the workspace and at most 1024 per
+// (query, head).
+size_t vectorChunks(const AttnArgs &a, int d, bool int8, size_t ws_bytes) {
+    const int U = int8 ? 8 : 4;
+    const size_t tile = size_t(kWave / (d / 8)) * U * kWaves; // keys per block step
+    const size_t groups = a.seq * size_t(a.nkvh) * size_t(a.group / sliceOf(a.group));
+    if (groups >= 512 || a.total <= tile) return 1;
+    const size_t n = std::min<size_t>((a.total + tile - 1) / tile, 1024);
+    const size_t per = size_t(d + 2) * sizeof(float) * a.seq * size_t(a.nh);
+    return std::max<size_t>(1, std::min(n, ws_bytes / per));
 }
 
 template <typename T, bool kInt8>
@@ -1225,23 +1240,13 @@ void launch(AttnArgs a, int d, int dv, void *ws, size_t ws_bytes, hipStream_t s)
             return;
         }
     }
-    // A block's waves each take one step of keys per chunk when the launch is split: about
-    // 2048 waves for decode, partials within the workspace and at most 1024 per (query, head).
-    const int U = kInt8 ? 8 : 4;
-    const size_t tile = size_t(kWave / (d / 8)) * U * kWaves; // keys per block step
-    const size_t groups = a.seq * size_t(a.nkvh) * size_t(a.slices);
-    size_t nchunks = 1;
-    if (groups < 512 && a.total > tile) {
-        nchunks = std::min<size_t>((a.total + tile - 1) / tile, 1024);
-        const size_t per = size_t(d + 2) * sizeof(float) * a.seq * size_t(a.nh);
-        nchunks = std::max<size_t>(1, std::min(nchunks, ws_bytes / per));
-    }
+    const size_t nchunks = vectorChunks(a, d, kInt8, ws_bytes);
     a.nchunks = int(nchunks);
     a.chunk = int(std::min<size_t>(nchunks == 1 ? std::max<size_t>(a.total, 1)
                                                 : (a.total + nchunks - 1) / nchunks,
                                    size_t(INT32_MAX)));
     a.part = static_cast<float *>(ws);
-    const size_t blocks = groups * nchunks;
+    const size_t blocks = a.seq * size_t(a.nkvh) * size_t(a.slices) * nchunks;
     if (d == 64)
         launchD<T, kInt8, 64>(a, G, blocks, s);
     else
@@ -1261,6 +1266,22 @@ void dispatch(AttnArgs a, int d, int dv, llaisysDataType_t dt, void *ws, size_t 
 }
 
 } // namespace
+
+extern "C" void llaisysTestAttentionRoute(size_t seq, size_t total, size_t nh, size_t nkvh, size_t d, int int8, int dt, int route[4]) {
+    AttnArgs a{};
+    a.seq = seq;
+    a.total = total;
+    a.nh = int(nh);
+    a.nkvh = int(nkvh);
+    a.group = int(nh / nkvh);
+    a.scale = 1.0f;
+    Prefill p{};
+    const bool takes = planPrefill(p, a, int(d), int(d), int8 != 0, llaisysDataType_t(dt));
+    route[0] = takes;
+    route[1] = takes ? p.nchunks : 0;
+    route[2] = takes ? p.chunk : 0;
+    route[3] = takes ? int(p.blocks) : 0;
+}
 
 // ---- scratch of the allocation-free entry point -----------------------------------------
 // File-scope device array holding the split attention's partials for
@@ -1309,12 +1330,19 @@ size_t selfAttentionInt8KVScratchBytes(const void *out, const void *q, const voi
     a.nkvh = int(nkvh);
     a.group = int(nh / nkvh);
     a.scale = scale;
-    Prefill p;
-    if (seq > 0 && nh > 0 && dt == LLAISYS_DTYPE_BF16 && d == 128 && planPrefill(p, a, int(d), int(dv), true, dt)) {
-        const size_t part = (p.part_bytes + 255) / 256 * 256, cache = 2 * total * nkvh * d * sizeof(uint16_t);
-        return part + cache <= cap ? part + cache : part;
+    const size_t most = selfAttentionWorkspaceBytes(seq, nh, d);
+    // a bf16 prefill with head_dim 128 is always accepted
+    if (nh > 0 && dt == LLAISYS_DTYPE_BF16 && d == 128 && seq >= size_t(kMfmaQ) && total > 0 && scale > 0.0f &&
+        std::isfinite(scale) && vecShape(a, int(d), int(dv), true)) {
+        Prefill p;
+        if (planPrefill(p, a, int(d), int(dv), true, dt)) {
+            const size_t part = (p.part_bytes + 255) / 256 * 256, cache = 2 * total * nkvh * d * sizeof(uint16_t);
+            return part + cache <= cap ? part + cache : part;
+        }
+        const size_t n = vectorChunks(a, int(d), true, most);
+        return n > 1 ? std::min(cap, n * seq * nh * (d + 2) * sizeof(float)) : 0;
     }
-    return selfAttentionWorkspaceBytes(seq, nh, d);
+    return most;
 }
 
 size_t selfAttentionWorkspaceBytes(size_t seq, size_t nh, size_t head_dim) {
