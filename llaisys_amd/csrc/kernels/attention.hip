@@ -18,10 +18,12 @@
 //  - attnPrefill (bf16 / f16, head_dim 64 or 128, >= 16 queries): 32 queries of two q heads per
 //    block on v_mfma_f32_32x32x16, the keys split over the block's waves and, where the blocks
 //    leave CUs idle, over blocks (merged by attnCombineFew / attnCombine).
+//  - attnPrefill16 (bf16, head_dim 128, >= 16 queries): 16 queries of 1, 2 or 4 q heads per block on
+//    v_mfma_f32_16x16x32, for the calls that are over before attnPrefill's larger blocks pay (planPrefill).
 //  - attnDecodeMfma (bf16 q, head_dim 128, fewer queries: decode, cache in bf16 or INT8):
 //    HBM-bound; the key range is cut into chunks, one block per (query, kv head, chunk) with
 //    the kv head's q heads as the MFMA columns; attnCombine merges the chunk partials.
-//  - attnGroup (f32, fewer queries in f16 or with head_dim 64): one wavefront per q head, the
+//  - attnGroup (f32, fewer queries in f16 or with head_dim 64, and short prefills of these): one wavefront per q head, the
 //    waves of a block being q heads of one kv head (they read the same K / V rows).  A key row of D elements
 //    is spread over R = D / 8 lanes, 8 elements per lane, so one load instruction covers
 //    64 / R keys; per batch of U instructions the wave forms its scores (8 FMAs, a butterfly
@@ -208,6 +210,11 @@ __global__ void __launch_bounds__(kWave * kWaves)
             m[j] = mx;
 #pragma unroll
             for (int u = 0; u < U; ++u) s[j][u] = s[j][u] == -INFINITY ? 0.0f : __expf(s[j][u] - mx);
+        }
+        if (kb + TILE > k1) { // the filler rows weigh 0, and 0 * Inf would not be 0
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (!ok[u]) vr[u] = typename IO::Raw{}, vsc[u] = 0.0f;
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -835,6 +842,244 @@ __global__ void __launch_bounds__(kWave * 2 * kSplits, 2)
     }
 }
 
+// ---- prefill of few heads per kv head: 16 queries per block (bf16, head_dim 128) -------------
+// A block takes 16 queries of W q heads of one kv head, a wave each (kSplit: two, each walking half
+// of the 64-key tiles), on v_mfma_f32_16x16x32: S^T = K Q^T in 4 score tiles per step, lane (n, g4) with
+// the scores of query n, then O^T += V^T P^T with P in two bf16 parts as attnPrefill's.  A[m = l % 16]
+// [k = 8 (l / 16) + j], B[k = 8 (l / 16) + j][n = l % 16], D[m = 4 (l / 16) + i][n = l % 16]; row m of
+// score tile t is key 32 (t / 2) + 8 (m / 4) + 4 (t % 2) + m % 4, so lane group g4 holds the 8
+// consecutive keys its part of the P V product takes.  Tiles come by global_load_lds_dwordx4 in two
+// stages, chunks swizzled by swzK / swzV.
+constexpr int kTileKeys = 64;
+__device__ __forceinline__ int swzK(int r) { return (r & 3) | (((r >> 3) & 3) << 2); }
+
+template <int W>
+__global__ void __launch_bounds__(kWave * W * 2)
+    attnPrefill16(AttnArgs a) {
+    constexpr int D = 128, KB = D / 32, DT = D / 16;
+    constexpr int kRowB = 2 * D;               // bytes of a key row
+    constexpr int kTileB = kTileKeys * kRowB;  // one K or V tile
+    constexpr int kLoads = 2 * kTileB / 1024;  // 1 KB load instructions per stage
+    constexpr int kPer = (kLoads + W - 1) / W;
+    __shared__ __align__(16) char lds_all[2][2][2 * kTileB]; // [half][stage][K tile | V tile]
+    const int wave_all = __builtin_amdgcn_readfirstlane(int(threadIdx.x) / kWave);
+    const int half = wave_all / W, wave = wave_all % W;
+    const int lane = int(threadIdx.x) % kWave;
+    const int n = lane % 16, g4 = lane / 16;
+
+    const size_t nqb = (a.seq + 15) / 16;
+    unsigned b = blockIdx.x;
+    const int sl = int(b % unsigned(a.slices));
+    b /= unsigned(a.slices);
+    const int g = int(b % unsigned(a.nkvh));
+    const size_t qb = nqb - 1 - size_t(b / unsigned(a.nkvh)); // latest queries first
+    const int h = g * a.group + sl * W + wave;
+    const size_t q0 = qb * 16;
+    const size_t qi = min(q0 + size_t(n), a.seq - 1);
+    const size_t vis_q = visibleKeys(a.total, a.seq, qi);
+    size_t most, least;
+    visibleRange(a.total, a.seq, q0, min(q0 + 15, a.seq - 1), most, least);
+    const size_t ntiles = (most + kTileKeys - 1) / kTileKeys;
+    const float c2 = a.scale * 1.4426950408889634f;
+
+    bf16x8 qreg[KB];
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+        const uint16_t *qp = static_cast<const uint16_t *>(a.q) + (qi * a.nh + h) * D + 32 * kb + 8 * g4;
+        qreg[kb] = asBf16x8(*reinterpret_cast<const v4u *>(qp));
+    }
+    float m = -INFINITY, lsum = 0.0f;
+    f32x4 o[DT];
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) o[dt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+
+    // load instruction j of this wave is stage load q = wave + W j (K rows for q < 16, then
+    // V rows): rows 4 (q % 16) + lane / 16 of the tile, LDS slot lane % 16 receiving chunk
+    // slot ^ swizzle(row) of the kv head's row
+    const size_t rowB = size_t(a.nkvh) * kRowB; // bytes between consecutive keys
+    const char *cache[2] = {static_cast<const char *>(a.k), static_cast<const char *>(a.v)};
+    // (byte offsets within a tile fit 32 bits: the launcher checks 64 rows * rowB < 2^31)
+    int lrow[kPer];
+    uint32_t loff[kPer], lcol[kPer];
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+        const int q = wave + W * j;
+        const int row = 4 * (q % 16) + lane / 16, slot = lane % 16;
+        const int chunk = slot ^ (q < 16 ? swzK(row) : swzV(row));
+        lrow[j] = row;
+        lcol[j] = uint32_t(g * kRowB + chunk * 16);
+        loff[j] = uint32_t(row) * uint32_t(rowB) + lcol[j];
+    }
+    const auto issue = [&](size_t t0, int stage) {
+        char *dst = &lds_all[half][stage][0];
+        const size_t left = a.total - t0; // keys of the cache from t0 on (> 0)
+        const bool full = left >= size_t(kTileKeys);
+#pragma unroll
+        for (int j = 0; j < kPer; ++j) {
+            const int q = wave + W * j;
+            if (q >= kLoads) break;
+            // the tile's rows from the tile base; in the cache's last tile, rows past it read row 0
+            const char *src = full || size_t(lrow[j]) < left ? cache[q / 16] + t0 * rowB + loff[j]
+                                                            : cache[q / 16] + lcol[j];
+            __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1))) *)(src),
+                                             (void __attribute__((address_space(3))) *)(dst + q * 1024), 16, 0, 0);
+        }
+    };
+
+    const size_t nsteps = (ntiles + 1) / 2;
+    const size_t tbeg = half ? nsteps : 0;
+    const size_t tcount = half ? ntiles - nsteps : nsteps;
+    if (tcount > 0) issue(tbeg * kTileKeys, 0);
+    for (size_t it = 0; it < nsteps; ++it) {
+        const int buf = int(it & 1);
+        const size_t kt0 = (tbeg + it) * kTileKeys;
+        waitVmcnt<0>(); // this wave's loads of tile it have landed
+        ldsBarrier();   // every wave's have; every wave is past the step that read the other stage
+        if (it + 1 < tcount) issue(kt0 + kTileKeys, buf ^ 1);
+        if (it >= tcount) continue;
+        const char *kt = &lds_all[half][buf][0], *vt = kt + kTileB;
+        const bool whole = kt0 + kTileKeys <= least;
+        const int nvis = int(min(vis_q - min(vis_q, kt0), size_t(kTileKeys)));
+        float p[4][4];
+        float mx = m;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const int krow = 32 * (t / 2) + 8 * (n / 4) + 4 * (t % 2) + n % 4; // A row n
+            const char *kr = kt + krow * kRowB;
+            const int sw = swzK(krow);
+            f32x4 acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int kb = 0; kb < KB; ++kb) {
+                const v4u kv = *reinterpret_cast<const v4u *>(kr + 16 * ((4 * kb + g4) ^ sw));
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(asBf16x8(kv), qreg[kb], acc, 0, 0, 0);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) p[t][i] = acc[i];
+        }
+        if (!whole) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int off = 32 * (t / 2) + 8 * g4 + 4 * (t % 2) + i;
+                    p[t][i] = off < nvis ? p[t][i] : -INFINITY;
+                }
+        }
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) mx = fmaxf(mx, p[t][i]);
+        mx = fmaxf(mx, __shfl_xor(mx, 16, kWave));
+        mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
+        const float mc = mx == -INFINITY ? 0.0f : mx * c2;
+        float ps = 0.0f;
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                p[t][i] = __builtin_amdgcn_exp2f(__builtin_fmaf(p[t][i], c2, -mc));
+                ps += p[t][i];
+            }
+        if (__builtin_expect(__any(mx != m), 0)) {
+            const float corr = mx == m ? 1.0f : __builtin_amdgcn_exp2f(__builtin_fmaf(m, c2, -mc));
+            lsum *= corr;
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) o[dt] *= corr;
+        }
+        m = mx;
+        lsum += ps;
+        // the transposing reads' rows and column offset: keys 32 p2 + 8 g + n / 4 (and + 4),
+        // columns 16 dt + 4 (n % 4) .. + 3, i.e. half n % 2 of chunk 2 dt + (n % 4) / 2
+#pragma unroll
+        for (int p2 = 0; p2 < 2; ++p2) {
+            uint32_t hw[4], lw[4];
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                const float x0 = p[2 * p2 + w / 2][2 * (w % 2)], x1 = p[2 * p2 + w / 2][2 * (w % 2) + 1];
+                splitPair<BF16>(x0, x1, hw[w], lw[w]);
+            }
+            const bf16x8 bhi = asBf16x8(v4u{hw[0], hw[1], hw[2], hw[3]});
+            const bf16x8 blo = asBf16x8(v4u{lw[0], lw[1], lw[2], lw[3]});
+            const int r0 = 32 * p2 + 8 * g4 + n / 4;
+            const char *v0 = vt + r0 * kRowB + 8 * (n % 2), *v1 = v0 + 4 * kRowB;
+            const int sw = swzV(r0); // rows r0 and r0 + 4 share it
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) {
+                const int cofs = 16 * ((2 * dt + (n % 4) / 2) ^ sw);
+                const uint64_t e0 = ldsReadTr16(v0 + cofs), e1 = ldsReadTr16(v1 + cofs);
+                const v4u vv = v4u{uint32_t(e0), uint32_t(e0 >> 32), uint32_t(e1), uint32_t(e1 >> 32)};
+                o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(asBf16x8(vv), bhi, o[dt], 0, 0, 0);
+                o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(asBf16x8(vv), blo, o[dt], 0, 0, 0);
+            }
+        }
+    }
+    float lt = lsum + __shfl_xor(lsum, 16, kWave);
+    lt += __shfl_xor(lt, 32, kWave);
+    float *xch = reinterpret_cast<float *>(&lds_all[0][0][0]) + size_t(wave) * kWave * (2 + 4 * DT);
+    __syncthreads();
+    if (half == 1) {
+        xch[lane] = m;
+        xch[kWave + lane] = lt;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) xch[(2 + 4 * dt + i) * kWave + lane] = o[dt][i];
+    }
+    __syncthreads();
+    if (half == 1) return;
+    const float m1 = xch[lane], l1 = xch[kWave + lane];
+    const float M = fmaxf(m, m1);
+    const float f0 = m == M ? 1.0f : __builtin_amdgcn_exp2f(__builtin_fmaf(m, c2, -M * c2));
+    const float f1 = m1 == M ? 1.0f : __builtin_amdgcn_exp2f(__builtin_fmaf(m1, c2, -M * c2));
+    lt = lt * f0 + l1 * f1;
+    m = M;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[dt][i] = o[dt][i] * f0 + xch[(2 + 4 * dt + i) * kWave + lane] * f1;
+    // as attnPrefill: a query whose outputs are not finite though its weights are is summed again over
+    // its own keys, 64 columns at a time
+    const bool live = q0 + size_t(n) < a.seq;
+    float z = 0.0f;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) z = __builtin_fmaf(o[dt][i], 0.0f, z);
+    const uint64_t redo = __ballot(live && z != z && lt == lt);
+    if (__builtin_expect(redo != 0, 0)) {
+        const float mc = m == -INFINITY ? 0.0f : m * c2;
+        uint32_t rows = uint32_t(redo | redo >> 16 | redo >> 32 | redo >> 48) & 0xFFFFu;
+        while (rows) {
+            const int r = __builtin_ctz(rows);
+            rows &= rows - 1;
+            const size_t i = q0 + size_t(r);
+            const uint16_t *qrow = static_cast<const uint16_t *>(a.q) + (i * a.nh + h) * D;
+#pragma unroll
+            for (int ch = 0; ch < 2; ++ch) {
+                const float y = visibleSum<BF16, false, D>(a, qrow, g, kWave * ch + lane, 0, visibleKeys(a.total, a.seq, i), c2,
+                                                           __shfl(mc, r, kWave));
+#pragma unroll
+                for (int dt = 0; dt < DT / 2; ++dt)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float ye = __shfl(y, 16 * dt + 4 * g4 + e, kWave);
+                        f32x4 &od = o[DT / 2 * ch + dt];
+                        od[e] = n == r ? ye : od[e];
+                    }
+            }
+        }
+    }
+    if (!live) return;
+    const float inv = lt == 0.0f ? 0.0f : 1.0f / lt;
+    uint16_t *op = static_cast<uint16_t *>(a.out) + (qi * a.nh + h) * D + 4 * g4;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) {
+        const uint32_t w0 = f32ToBf16(o[dt][0] * inv) | (f32ToBf16(o[dt][1] * inv) << 16);
+        const uint32_t w1 = f32ToBf16(o[dt][2] * inv) | (f32ToBf16(o[dt][3] * inv) << 16);
+        *reinterpret_cast<v2u *>(op + 16 * dt) = v2u{w0, w1};
+    }
+}
+
 // Merge of few chunk partials for many (query, head) pairs: a thread per 4 columns of a pair.
 // (attnCombine spends 1024 threads on 32 columns of a pair, for up to 1024 chunks.)
 template <typename T>
@@ -1087,10 +1332,12 @@ int sliceOf(int group) {
     return 1;
 }
 
+// Load instructions per step of the vector kernel: 16 bytes of K and V codes per lane, or 32 of elements
+constexpr int groupLoads(bool int8) { return int8 ? 8 : 4; }
+
 template <typename T, bool kInt8, int D, int G>
 void launchGroup(const AttnArgs &a, size_t blocks, hipStream_t s) {
-    constexpr int U = kInt8 ? 8 : 4; // 16 bytes of K and V codes per lane per step, or 32 of elements
-    attnGroup<T, kInt8, D, G, U><<<unsigned(blocks), kWave * kWaves, 0, s>>>(a);
+    attnGroup<T, kInt8, D, G, groupLoads(kInt8)><<<unsigned(blocks), kWave * kWaves, 0, s>>>(a);
 }
 
 template <typename T, bool kInt8, int D>
@@ -1111,47 +1358,11 @@ bool vecShape(const AttnArgs &a, int d, int dv, bool int8) {
            (int8 ? aligned(a.k, 8) && aligned(a.v, 8) : aligned(a.k, 16) && aligned(a.v, 16));
 }
 
-// The prefill on MFMA: bf16 or f16, head_dim 64 or 128, 16 or more queries, a non-empty cache and
-// a positive finite scale (the kernel tracks the max of the raw dot products).
-struct Prefill {
-    int slices, chunk, nchunks;
-    size_t blocks, part_bytes;
-    bool heads; // the block's units are two q heads (else two 32-query blocks of one head)
-};
-constexpr size_t kPrefillPartBytes = size_t(8) << 20;
-
-// How the prefill is cut; false where it does not apply.  Depends on the shape only, so that every
-// entry point sums a shape in the same order.  Keys are split over blocks where the query blocks
-// alone would leave CUs idle, into chunks of at least 4 steps (512 keys): 16 queries over 32768
-// keys would otherwise be 256 steps in each of 6 blocks.
-bool planPrefill(Prefill &p, const AttnArgs &a, int d, int dv, bool int8, llaisysDataType_t dt) {
-    if ((dt != LLAISYS_DTYPE_BF16 && dt != LLAISYS_DTYPE_F16) || !vecShape(a, d, dv, int8)) return false;
-    if (a.total == 0 || a.seq < size_t(kMfmaQ) || !(a.scale > 0.0f) || !std::isfinite(a.scale)) return false;
-    // the kernel's lane offsets within one 1 KB load (512 / d key rows) have 32 bits
-    if (size_t(a.nkvh) * 1024 >= size_t(1) << 32) return false;
-    p.heads = a.group % 2 == 0;
-    p.slices = p.heads ? a.group / 2 : a.group;
-    const size_t qb = (a.seq + (p.heads ? 31 : 63)) / (p.heads ? 32 : 64);
-    p.blocks = qb * size_t(a.nkvh) * size_t(p.slices);
-    const size_t steps = (a.total + kStepKeys - 1) / kStepKeys;
-    const size_t cap = kPrefillPartBytes / (a.seq * size_t(a.nh) * size_t(d + 2) * sizeof(float));
-    size_t n = std::max<size_t>(1, std::min({256 / p.blocks, steps / 4, cap, size_t(1024)}));
-    const size_t per = (steps + n - 1) / n;
-    n = (steps + per - 1) / per;
-    if (per * kStepKeys > size_t(INT32_MAX)) return false;
-    p.chunk = int(per * kStepKeys);
-    p.nchunks = int(n);
-    p.part_bytes = n > 1 ? a.seq * size_t(a.nh) * n * size_t(d + 2) * sizeof(float) : 0;
-    p.blocks *= n;
-    return p.blocks < (size_t(1) << 31);
-}
-
-// Chunks of the vector kernel's keys.  A block's waves each take one step of keys per chunk when the
-// launch is split: about 2048 waves for decode, partials within the workspace and at most 1024 per
+// Chunks of the vector kernel's keys.  A block's waves each take one step of keys (U loads) per chunk when
+// the launch is split: about 2048 waves for decode, partials within the workspace and at most 1024 per
 // (query, head).
-size_t vectorChunks(const AttnArgs &a, int d, bool int8, size_t ws_bytes) {
-    const int U = int8 ? 8 : 4;
-    const size_t tile = size_t(kWave / (d / 8)) * U * kWaves; // keys per block step
+size_t vectorChunks(const AttnArgs &a, int d, int U, size_t ws_bytes) {
+    const size_t tile = size_t(kWave / (d / 8)) * size_t(U) * kWaves; // keys per block step
     const size_t groups = a.seq * size_t(a.nkvh) * size_t(a.group / sliceOf(a.group));
     if (groups >= 512 || a.total <= tile) return 1;
     const size_t n = std::min<size_t>((a.total + tile - 1) / tile, 1024);
@@ -1159,18 +1370,187 @@ size_t vectorChunks(const AttnArgs &a, int d, bool int8, size_t ws_bytes) {
     return std::max<size_t>(1, std::min(n, ws_bytes / per));
 }
 
+// Expected time in us of a launch of one block per CU at a time: the launch, and for each block `block` and,
+// per 128 keys, `step` + `busy` times the share of CUs that have one.  The blocks with the most keys
+// start first; of more than kCUs blocks, the longest that starts second starts after the shortest of
+// the first kCUs.
+constexpr double kLaunchUs = 2.4;
+constexpr int kCUs = 256;
+struct BlockTime {
+    double block, step, busy;
+    double stepUs(size_t blocks) const { return step + busy * std::min(1.0, double(blocks) / kCUs); }
+};
+double roundsUs(const BlockTime &t, size_t blocks, size_t longest, size_t shortest) {
+    const double full = double(blocks) / kCUs, lo = double(shortest), hi = double(longest), step = t.stepUs(blocks);
+    double us = t.block + step * hi;
+    // (1.07: rounds do not follow on each other without a gap)
+    if (full > 1.0)
+        us = std::max({us, 1.07 * full * (t.block + step * (lo + hi) / 2), 1.07 * 2 * (t.block + step * (hi - (hi - lo) / full))});
+    return kLaunchUs + us;
+}
+
+// How a call of 16 or more queries runs (bf16 or f16, head_dim 64 or 128, a non-empty cache and a
+// positive finite scale: the MFMA kernels track the max of the raw dot products).
+enum class PrefillKernel { k32, k16, kGroup, kGroup8 }; // attnPrefill, attnPrefill16, attnGroup with 4 and 8 loads per step
+struct Prefill {
+    PrefillKernel kernel;
+    int heads;     // q heads per block; attnPrefill: 2, or 1 of 64 queries
+    int chunk, nchunks;
+    size_t blocks, part_bytes;
+    bool elements; // an INT8 cache is dequantized into the workspace first
+    size_t need;   // bytes of workspace it cannot do without
+};
+constexpr size_t kPrefillPartBytes = size_t(8) << 20;
+
+// attnPrefill's times by type, head_dim and cache (Codes: INT8 converted in the kernel), with those of
+// a launch whose keys are split: a chunk's merge and its 10000 partials.  From sweeps over 16 to 512
+// (bf16, 128: 2048) queries, 0 to 1600 (4096) earlier keys and ten head counts; rms error 3 to 5%.
+struct PrefillTime {
+    BlockTime t;
+    double merge, partials;
+};
+constexpr PrefillTime kBf16D128{{4.32, 1.62, 0.32}, 0.88, 3.4}, kBf16D128Codes{{3.96, 2.29, 0.18}, 0.84, 3.2};
+constexpr PrefillTime kBf16D64{{2.78, 1.20, 0.24}, 1.10, 1.5}, kBf16D64Codes{{2.63, 1.51, 0.19}, 1.10, 1.5};
+constexpr PrefillTime kF16D128{{5.17, 1.60, 0.51}, 0.77, 2.9}, kF16D64{{4.15, 1.19, 0.24}, 0.72, 1.4};
+// attnPrefill16 with 1, 2 and 4 heads per block; rms error 2 to 3%
+constexpr BlockTime kTiles16[3] = {{2.03, 1.95, 0.0}, {2.07, 1.62, 0.04}, {2.82, 1.68, 0.13}};
+// attnGroup over elements with 1 and 2 heads per block (more heads, and f16 with head_dim 64, are slower
+// than attnPrefill at every size measured): a launch, a round of kCUs blocks, 100000 block keys, a key tile, and split as above
+struct GroupTime {
+    double base, round, keys, tile, merge, partials;
+};
+constexpr GroupTime kGroupBf16D64[2] = {{1.09, 0.70, 1.12, 0.24, 3.6, 15.2}, {1.25, 1.46, 0.98, 0.95, 2.9, 23.7}};
+constexpr GroupTime kGroupF16D128[2] = {{3.39, 1.60, 6.41, 1.06, 3.1, 42.7}, {3.60, 2.75, 0.0, 2.45, 2.5, 60.0}};
+
+// Dequantizing an INT8 cache of `el` elements (K and V): a launch, which small caches are not much more than
+double dequantizeUs(size_t el) {
+    const double m = double(el) * 1e-6;
+    return 2.0 + std::min(5.0 * m, 3.0 + 1.3 * m);
+}
+
+// How the prefill is cut; false where it does not apply.  Kernel and cut depend on the shape only, not
+// on the entry point or on how the cache is kept, so that all of them give the same bits.
+//  - attnPrefill: keys are split over blocks where the query blocks alone would leave CUs idle, into
+//    chunks of at least 4 steps (512 keys): 16 queries over 32768 keys would otherwise be 256 steps in
+//    each of 6 blocks.
+//  - Its block costs about 4 us beside its steps, so calls of few steps and of less than two rounds of
+//    small blocks run faster on attnPrefill16 (bf16, 128; 100 queries, 32 / 8 heads 8.4 -> 6.5 us) or
+//    attnGroup (16 queries, 16 / 16 heads of 64, bf16 5.7 -> 4.0 us).
+//  - attnPrefill converts a bf16 INT8 cache in the kernel until the query blocks that convert a tile again
+//    cost more than one launch that dequantizes it (16 / 16 heads of 128, 64 queries over 1264 keys 28.8 ->
+//    21.0 us; from about 3000 queries the other way round).  f16 codes cost five times as much.
+bool planPrefill(Prefill &p, const AttnArgs &a, int d, int dv, bool int8, llaisysDataType_t dt) {
+    const bool bf16 = dt == LLAISYS_DTYPE_BF16;
+    if ((!bf16 && dt != LLAISYS_DTYPE_F16) || !vecShape(a, d, dv, int8)) return false;
+    if (a.total == 0 || a.seq < size_t(kMfmaQ) || !(a.scale > 0.0f) || !std::isfinite(a.scale)) return false;
+    // the kernel's lane offsets within one 1 KB load (512 / d key rows) have 32 bits
+    if (size_t(a.nkvh) * 1024 >= size_t(1) << 32) return false;
+    const size_t nh = size_t(a.nh), bq = a.group % 2 == 0 ? 32 : 64;
+    p.kernel = PrefillKernel::k32;
+    p.heads = a.group % 2 == 0 ? 2 : 1;
+    p.blocks = (a.seq + bq - 1) / bq * (nh / p.heads);
+    const size_t steps = (a.total + kStepKeys - 1) / kStepKeys;
+    const size_t partial = a.seq * nh * size_t(d + 2) * sizeof(float);
+    size_t n = std::max<size_t>(1, std::min({256 / p.blocks, steps / 4, kPrefillPartBytes / partial, size_t(1024)}));
+    const size_t per = (steps + n - 1) / n;
+    n = (steps + per - 1) / per;
+    if (per * kStepKeys > size_t(INT32_MAX)) return false;
+    p.chunk = int(per * kStepKeys);
+
+    const size_t past = a.total > a.seq ? a.total - a.seq : 0;
+    const double partials = double(a.seq * nh) * 1e-4;
+    // steps of the block of the first q queries, the fewest
+    const auto first = [&](size_t q) { return (std::min(a.total, past + q) + kStepKeys - 1) / kStepKeys; };
+    const auto prefillUs = [&](const PrefillTime &t) {
+        // (odd groups, up to 32 queries: the second unit's queries are repeats)
+        if (n == 1) return (p.heads == 1 && a.seq <= 32 ? 0.9 : 1.0) * roundsUs(t.t, p.blocks, steps, first(bq));
+        return kLaunchUs + t.t.block + t.t.stepUs(p.blocks * n) * double(per) + (t.merge + t.partials * partials) * double(n);
+    };
+    double us = prefillUs(bf16 ? (d == 128 ? kBf16D128 : kBf16D64) : (d == 128 ? kF16D128 : kF16D64));
+    const size_t el = 2 * a.total * size_t(a.nkvh) * size_t(d), el_bytes = el * sizeof(uint16_t);
+    const double deq = dequantizeUs(el);
+    p.elements = int8 && !(bf16 && prefillUs(d == 128 ? kBf16D128Codes : kBf16D64Codes) < us + deq);
+    // attnPrefill16 reads elements only: caches that an INT8 call can dequantize, whichever entry point it has
+    const size_t ws = std::min(kNoAllocScratchBytes, selfAttentionWorkspaceBytes(a.seq, nh, size_t(d)));
+    if (bf16 && d == 128 && el_bytes <= ws && size_t(a.nkvh) * 256 * kTileKeys < size_t(1) << 31) {
+        for (int w : {4, 2, 1}) {
+            if (a.group % w != 0 || (w == 1 && a.group % 2 == 0)) continue;
+            const size_t blocks = (a.seq + 15) / 16 * (nh / size_t(w));
+            const double t = roundsUs(kTiles16[w / 2], blocks, steps, first(16));
+            if (blocks > 2 * kCUs || t >= us) continue;
+            us = t;
+            p.kernel = PrefillKernel::k16;
+            p.heads = w;
+            p.blocks = blocks;
+            p.elements = int8;
+        }
+    }
+    const int G = sliceOf(a.group);
+    if (bf16 == (d == 64) && G <= 2) {
+        const GroupTime &t = bf16 ? kGroupBf16D64[G - 1] : kGroupF16D128[G - 1];
+        const size_t groups = a.seq * (nh / size_t(G)), tile = size_t(kWave / (d / 8)) * groupLoads(false) * kWaves;
+        // one round of blocks over one to two tiles of keys: twice the loads per step and no split (64 queries
+        // over 464 keys, 4 / 4 heads, bf16 10.1 -> 5.8 us, INT8 11.3 -> 7.7 us)
+        const bool twice = bf16 && groups <= kCUs && a.total > tile && a.total <= 2 * tile;
+        const size_t c = twice ? 1 : vectorChunks(a, d, groupLoads(false), selfAttentionWorkspaceBytes(a.seq, nh, size_t(d)));
+        const double keys = double(a.total) - double(std::min(a.seq, a.total)) / 2;
+        const double tiles = double(a.total) / double(tile);
+        double g = kLaunchUs + t.base + t.round * std::ceil(double(groups * c) / kCUs) + t.keys * double(groups) * keys * 1e-5;
+        g += c > 1 ? t.tile + t.merge + t.partials * partials * double(c) : t.tile * (tiles < 1 ? tiles : std::ceil(tiles));
+        if ((twice || g < us) && groups * c < size_t(1) << 31) {
+            p.kernel = twice ? PrefillKernel::kGroup8 : PrefillKernel::kGroup;
+            p.heads = G;
+            p.blocks = groups;
+            p.chunk = int(c == 1 ? std::min<size_t>(a.total, size_t(INT32_MAX)) : (a.total + c - 1) / c);
+            n = c;
+            // 0.5 us and 1.5e-5 us per block and key is what the kernel takes longer over codes
+            p.elements = int8 && !twice && (!bf16 || 0.5 + 1.5e-5 * double(groups * a.total) > deq);
+        }
+    }
+    if (p.kernel == PrefillKernel::k16) n = 1;
+    p.nchunks = int(n);
+    p.blocks *= n;
+    p.part_bytes = n > 1 ? partial * n : 0;
+    p.need = int8 && p.kernel == PrefillKernel::k16 ? el_bytes : p.part_bytes;
+    return p.blocks < (size_t(1) << 31);
+}
+
+template <typename T, bool kInt8, int D>
+void launchPrefillKernel(const AttnArgs &a, const Prefill &p, hipStream_t s) {
+    const unsigned blocks = unsigned(p.blocks);
+    if (p.kernel == PrefillKernel::kGroup8) {
+        if constexpr (std::is_same_v<T, BF16> && D == 64)
+            p.heads == 2 ? attnGroup<T, kInt8, D, 2, 8><<<blocks, kWave * kWaves, 0, s>>>(a)
+                         : attnGroup<T, kInt8, D, 1, 8><<<blocks, kWave * kWaves, 0, s>>>(a);
+    } else if (p.kernel == PrefillKernel::kGroup) {
+        // (the loads per step of elements also for codes, so that both sum in the same order)
+        if constexpr (std::is_same_v<T, F16> == (D == 128))
+            p.heads == 2 ? attnGroup<T, kInt8, D, 2, groupLoads(false)><<<blocks, kWave * kWaves, 0, s>>>(a)
+                         : attnGroup<T, kInt8, D, 1, groupLoads(false)><<<blocks, kWave * kWaves, 0, s>>>(a);
+    } else if (p.kernel == PrefillKernel::k16) {
+        if constexpr (std::is_same_v<T, BF16> && !kInt8 && D == 128) {
+            switch (p.heads) {
+            case 4: attnPrefill16<4><<<blocks, kWave * 8, 0, s>>>(a); return;
+            case 2: attnPrefill16<2><<<blocks, kWave * 4, 0, s>>>(a); return;
+            default: attnPrefill16<1><<<blocks, kWave * 2, 0, s>>>(a); return;
+            }
+        }
+    } else {
+        constexpr unsigned threads = kWave * 2 * kSplits;
+        p.heads == 2 ? attnPrefill<T, kInt8, D, true><<<blocks, threads, 0, s>>>(a)
+                     : attnPrefill<T, kInt8, D, false><<<blocks, threads, 0, s>>>(a);
+    }
+}
+
 template <typename T, bool kInt8>
 void launchPrefill(const AttnArgs &a, const Prefill &p, int d, hipStream_t s) {
-    const unsigned blocks = unsigned(p.blocks), threads = kWave * 2 * kSplits;
     if (d == 128)
-        p.heads ? attnPrefill<T, kInt8, 128, true><<<blocks, threads, 0, s>>>(a)
-                : attnPrefill<T, kInt8, 128, false><<<blocks, threads, 0, s>>>(a);
+        launchPrefillKernel<T, kInt8, 128>(a, p, s);
     else
-        p.heads ? attnPrefill<T, kInt8, 64, true><<<blocks, threads, 0, s>>>(a)
-                : attnPrefill<T, kInt8, 64, false><<<blocks, threads, 0, s>>>(a);
+        launchPrefillKernel<T, kInt8, 64>(a, p, s);
     if (p.nchunks == 1) return;
     const size_t pairs = a.seq * size_t(a.nh);
-    if (p.nchunks <= 16)
+    if (p.nchunks <= 16 && p.kernel != PrefillKernel::kGroup)
         attnCombineFew<T><<<unsigned((pairs * size_t(d / 4) + 255) / 256), 256, 0, s>>>(a.out, a.part, p.nchunks, d, pairs);
     else
         launchCombine<T>(a.out, a.part, p.nchunks, d, pairs, s);
@@ -1190,17 +1570,17 @@ void launch(AttnArgs a, int d, int dv, void *ws, size_t ws_bytes, hipStream_t s)
     if constexpr (!std::is_same_v<T, F32>) {
         constexpr auto dt = std::is_same_v<T, BF16> ? LLAISYS_DTYPE_BF16 : LLAISYS_DTYPE_F16;
         Prefill p;
-        if (planPrefill(p, a, d, dv, kInt8, dt) && p.part_bytes <= ws_bytes) {
-            a.slices = p.slices;
+        if (planPrefill(p, a, d, dv, kInt8, dt) && p.need <= ws_bytes) {
+            a.slices = a.group / p.heads;
             a.chunk = p.chunk;
             a.nchunks = p.nchunks;
             a.part = static_cast<float *>(ws);
             if constexpr (kInt8) {
-                // An INT8 cache whose 16-bit form fits the workspace behind the partials is
-                // dequantized once (both caches in one launch, T(code * scale) as the tiles would be
-                // staged), so that the tiles of every query block no longer convert the same codes.
+                // Both caches in one launch, T(code * scale) as the tiles would be staged: the same
+                // operands, the same bits.  A cache whose 16-bit form does not fit the workspace behind
+                // the partials is converted in the kernel.
                 const size_t cache_el = a.total * size_t(a.nkvh) * size_t(d), off = (p.part_bytes + 255) / 256 * 256;
-                if (off + 2 * cache_el * sizeof(uint16_t) <= ws_bytes) {
+                if (p.elements && off + 2 * cache_el * sizeof(uint16_t) <= ws_bytes) {
                     uint16_t *kd = reinterpret_cast<uint16_t *>(static_cast<char *>(ws) + off), *vd = kd + cache_el;
                     dequantizeInt8Pair(kd, static_cast<const int8_t *>(a.k), a.ks, a.total * size_t(a.nkvh), vd,
                                        static_cast<const int8_t *>(a.v), a.vs, a.total * size_t(a.nkvh),
@@ -1240,7 +1620,7 @@ void launch(AttnArgs a, int d, int dv, void *ws, size_t ws_bytes, hipStream_t s)
             return;
         }
     }
-    const size_t nchunks = vectorChunks(a, d, kInt8, ws_bytes);
+    const size_t nchunks = vectorChunks(a, d, groupLoads(kInt8), ws_bytes);
     a.nchunks = int(nchunks);
     a.chunk = int(std::min<size_t>(nchunks == 1 ? std::max<size_t>(a.total, 1)
                                                 : (a.total + nchunks - 1) / nchunks,
@@ -1267,7 +1647,7 @@ void dispatch(AttnArgs a, int d, int dv, llaisysDataType_t dt, void *ws, size_t 
 
 } // namespace
 
-extern "C" void llaisysTestAttentionRoute(size_t seq, size_t total, size_t nh, size_t nkvh, size_t d, int int8, int dt, int route[4]) {
+extern "C" void llaisysTestAttentionRoute(size_t seq, size_t total, size_t nh, size_t nkvh, size_t d, int int8, int dt, int route[6]) {
     AttnArgs a{};
     a.seq = seq;
     a.total = total;
@@ -1277,10 +1657,12 @@ extern "C" void llaisysTestAttentionRoute(size_t seq, size_t total, size_t nh, s
     a.scale = 1.0f;
     Prefill p{};
     const bool takes = planPrefill(p, a, int(d), int(d), int8 != 0, llaisysDataType_t(dt));
-    route[0] = takes;
+    route[0] = takes ? 1 + int(p.kernel) : 0;
     route[1] = takes ? p.nchunks : 0;
     route[2] = takes ? p.chunk : 0;
     route[3] = takes ? int(p.blocks) : 0;
+    route[4] = takes ? p.heads : 0;
+    route[5] = takes && p.elements;
 }
 
 // ---- scratch of the allocation-free entry point -----------------------------------------
@@ -1337,9 +1719,9 @@ size_t selfAttentionInt8KVScratchBytes(const void *out, const void *q, const voi
         Prefill p;
         if (planPrefill(p, a, int(d), int(dv), true, dt)) {
             const size_t part = (p.part_bytes + 255) / 256 * 256, cache = 2 * total * nkvh * d * sizeof(uint16_t);
-            return part + cache <= cap ? part + cache : part;
+            return p.elements && part + cache <= cap ? part + cache : part;
         }
-        const size_t n = vectorChunks(a, int(d), true, most);
+        const size_t n = vectorChunks(a, int(d), groupLoads(true), most);
         return n > 1 ? std::min(cap, n * seq * nh * (d + 2) * sizeof(float)) : 0;
     }
     return most;

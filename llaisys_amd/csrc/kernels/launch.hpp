@@ -121,9 +121,10 @@ void selfAttention(void *out, const void *q, const void *k, const void *v, const
                    size_t d, size_t dv, float scale, llaisysDataType_t dt, void *ws,
                    size_t ws_bytes, hipStream_t stream);
 
-// How launch picks for head_dim 64 / 128, aligned, for the tests (no GPU needed): whether the MFMA
-// prefill takes the call, then its chunks, keys per chunk and blocks.
-extern "C" void llaisysTestAttentionRoute(size_t seq, size_t total, size_t nh, size_t nkvh, size_t d, int int8, int dt, int route[4]);
+// How launch picks for head_dim 64 / 128, aligned, for the tests (no GPU needed): 0 for the generic
+// launches, else 1 + PrefillKernel; the chunks, keys per chunk, blocks and q heads per block; whether an
+// INT8 cache is dequantized first.
+extern "C" void llaisysTestAttentionRoute(size_t seq, size_t total, size_t nh, size_t nkvh, size_t d, int int8, int dt, int route[6]);
 
 // out [rows, N] = x [rows, K] w^T (+ bias), w of N rows; with `scale` non-null w is INT8 codes and
 // the sum of each weight row n is multiplied by scale[n] (W8A16).  With `swiglu` w, scale and bias

@@ -1,4 +1,4 @@
-"""The MFMA prefill attention (attnPrefill) at the edges of its tiles, against the oracle: both
+"""The prefill attention (attnPrefill, attnPrefill16 and short calls on attnGroup) at the edges of its tiles, against the oracle: both
 16-bit types, both head dims, cache in the type and in INT8.  Tolerance: assert_attention_close."""
 import zlib
 
@@ -17,7 +17,12 @@ pytestmark = pytest.mark.gpu
 # query block of one query, even and odd groups (two heads / two query blocks per block), keys split
 # over blocks (few and many chunks), more queries than keys (the early ones wrap and see every key)
 EDGES = [(16, 16, 2, 1, 64), (33, 129, 4, 2, 128), (64, 97, 3, 1, 64), (65, 160, 5, 5, 128), (97, 384, 12, 2, 64),
-         (16, 4100, 12, 2, 128), (31, 20000, 3, 3, 64), (300, 200, 4, 2, 128), (130, 100, 3, 1, 64)]
+         (16, 4100, 12, 2, 128), (31, 20000, 3, 3, 64), (300, 200, 4, 2, 128), (130, 100, 3, 1, 64),
+         # bf16 on the 16-query kernel: one tile of 64 keys and one key more, an odd count of tiles (one wave set
+         # has one less), 1, 2 and 4 heads per block, queries past a block and wrapping queries; then
+         # attnGroup with 8 loads per step, and keys split over its blocks
+         (16, 64, 5, 1, 128), (17, 65, 8, 1, 128), (48, 129, 2, 2, 128), (270, 300, 32, 8, 128), (100, 60, 8, 2, 128),
+         (60, 400, 4, 4, 64), (24, 300, 8, 4, 64), (40, 1100, 2, 1, 64)]
 
 
 @pytest.mark.parametrize("dt", ["bf16", "f16"])
@@ -87,7 +92,7 @@ def visible_attention(q, k, v, scale):
 
 # seq, total, nh, nkvh: the diagonal within one step, rows past the cache in a part-filled tile, an odd
 # group's two query blocks, and keys split over blocks
-NON_FINITE = [(40, 40, 4, 2), (33, 201, 3, 1), (40, 1100, 2, 1)]
+NON_FINITE = [(40, 40, 4, 2), (33, 201, 3, 1), (40, 200, 12, 2), (40, 1100, 2, 1)]
 
 
 @pytest.mark.parametrize("int8", [False, True], ids=["plain", "int8"])
