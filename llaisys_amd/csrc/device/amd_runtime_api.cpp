@@ -12,6 +12,7 @@
 
 #include "../kernels/launch.hpp"
 
+#include <algorithm>
 #include <cstdlib>
 #include <memory>
 #include <mutex>
@@ -127,6 +128,8 @@ struct WsBuffer {
 struct WsSlots {
     std::shared_ptr<WsBuffer> buf[kMaxDevices];
     bool capturing[kMaxDevices] = {};
+    size_t refused[kMaxDevices] = {}; // size of tryWorkspace's last allocation that failed, 0 after a growth
+    unsigned tries[kMaxDevices] = {}; // calls since that asked for as much
 };
 // Never destroyed: at thread (and process) exit the HIP runtime may already be gone, so
 // the thread's buffers are left to the driver, as any device memory at exit.
@@ -135,16 +138,17 @@ WsSlots &wsSlots() {
     return *slots;
 }
 
-// Workspace reserved when a capture starts (bytes beyond the library's reserved head):
-// enough for every attention launch (its partials are capped at 64 MiB).  The environment
-// variable LLAISYS_GRAPH_WORKSPACE_BYTES overrides it.
+// Workspace reserved when a capture starts (bytes beyond the library's reserved head): enough for
+// every attention launch (its partials are capped at 64 MiB), and for the split sums of a linear
+// (48 MiB) behind 64 MiB of normalised rows, so that it sums in a graph as it does outside.  The
+// environment variable LLAISYS_GRAPH_WORKSPACE_BYTES overrides it.
 size_t captureReserve() {
     if (const char *e = std::getenv("LLAISYS_GRAPH_WORKSPACE_BYTES")) {
         char *end = nullptr;
         const unsigned long long v = std::strtoull(e, &end, 10);
         if (end != e && *end == '\0') return size_t(v);
     }
-    return size_t(64) << 20;
+    return size_t(112) << 20;
 }
 
 int currentDevice() {
@@ -192,20 +196,31 @@ void raiseIfError(llaisysStream_t s) {
 }
 
 namespace {
-// Moves the slot to a buffer of at least `bytes`, zeroed (kernels that keep a completion counter
-// in the workspace expect it zeroed once).  The old buffer is freed, after a device
-// synchronisation, once no graph holds it.
-int growWorkspace(std::shared_ptr<WsBuffer> &cur, size_t bytes, const char *&what) {
-    const size_t n = bytes < (size_t(1) << 20) ? (size_t(1) << 20) : bytes;
+// Moves the slot to a buffer of at least `bytes` and of half as much again as before (a first growth
+// stops the stream once, and sizes that rise step by step would stop it at each of them), its head
+// zeroed: kernels that keep a completion counter there expect that once.  The old buffer is freed,
+// after a device synchronisation, once no graph holds it.
+int growWorkspace(WsSlots &ws, int dev, size_t bytes, const char *&what) {
+    std::shared_ptr<WsBuffer> &cur = ws.buf[dev];
+    size_t n = std::max(bytes, size_t(1) << 20);
     void *p = nullptr;
     what = "hipMalloc(workspace)";
-    if (const int st = hipMalloc(&p, n)) return st;
+    const size_t more = cur ? cur->size + cur->size / 2 : 0;
+    if (more > n && hipMalloc(&p, more) == hipSuccess)
+        n = more;
+    else
+        p = nullptr;
+    if (!p) {
+        if (more > n) (void)hipGetLastError(); // no sticky error where the exact size is there
+        if (const int st = hipMalloc(&p, n)) return st;
+    }
     what = "hipMemset(workspace)";
-    if (const int st = hipMemset(p, 0, n)) {
+    if (const int st = hipMemset(p, 0, std::min(n, kernels::kScratchReserved))) {
         (void)hipFree(p);
         return st;
     }
     cur = std::make_shared<WsBuffer>(p, n);
+    ws.refused[dev] = 0;
     return hipSuccess;
 }
 } // namespace
@@ -224,7 +239,7 @@ void *workspace(int dev, size_t bytes) {
                                 "above that before llaisysGraphBeginCapture",
                          "workspace growth during capture");
         const char *what = nullptr;
-        const int st = growWorkspace(cur, bytes, what);
+        const int st = growWorkspace(ws, dev, bytes, what);
         check(st, what);
     }
     return cur->ptr;
@@ -237,14 +252,20 @@ void *tryWorkspace(int dev, size_t bytes, llaisysStream_t s) {
     if (!ws.capturing[dev]) {
         // a graph that the caller captures on the stream itself does not keep the buffer alive
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(static_cast<hipStream_t>(s), &cap) != hipSuccess || cap != hipStreamCaptureStatusNone)
+        if (hipStreamIsCapturing(static_cast<hipStream_t>(s), &cap) != hipSuccess) {
+            (void)hipGetLastError(); // as below: no sticky error for a call that does without
             return nullptr;
+        }
+        if (cap != hipStreamCaptureStatusNone) return nullptr;
     }
     if (cur && cur->size >= bytes) return cur->ptr;
     if (ws.capturing[dev]) return nullptr;
+    // memory that was not there a moment ago is asked for again every 256 calls
+    if (ws.refused[dev] && bytes >= ws.refused[dev] && ++ws.tries[dev] % 256) return nullptr;
     const char *what = nullptr;
-    if (growWorkspace(cur, bytes, what) != hipSuccess) {
+    if (growWorkspace(ws, dev, bytes, what) != hipSuccess) {
         (void)hipGetLastError(); // the caller goes on without: leave no sticky error
+        ws.refused[dev] = bytes;
         return nullptr;
     }
     return cur->ptr;
@@ -303,3 +324,9 @@ void destroyGraph(llaisysGraph_t g) {
 }
 
 } // namespace llaisys::device::amd
+
+// The calling thread's scratch on a device, in bytes, for the tests
+extern "C" __attribute__((visibility("default"))) size_t llaisysTestWorkspaceBytes(int dev) {
+    const auto &cur = llaisys::device::amd::wsSlots().buf[dev];
+    return cur ? cur->size : 0;
+}

@@ -121,8 +121,10 @@ Plan plan16(const LinearCall &c) {
 
 Plan planOf(const LinearCall &c) { return c.dt == LLAISYS_DTYPE_F32 ? planF32(c) : plan16(c); }
 
+// The partial sums of 2 N outputs with and without swiglu: where the scratch is short, gate / up in
+// one launch and its halves apart go without a split alike.
 size_t planBytes(const Plan &p, const LinearCall &c) {
-    return p.splits > 1 ? size_t(p.splits) * c.rows * (c.swiglu ? 2 * c.N : c.N) * sizeof(float) : 0;
+    return p.splits > 1 ? size_t(p.splits) * c.rows * 2 * c.N * sizeof(float) : 0;
 }
 
 template <bool kSw>

@@ -1,5 +1,6 @@
 """The tiled linear kernels (linear_gemm.hip) at the edges of their tiles and of their split of K,
 against the oracle's restatement of the reference linear.  Tolerance: numerics.assert_linear_close."""
+import ctypes
 import threading
 import zlib
 
@@ -9,6 +10,7 @@ import pytest
 import llaisys_amd as L
 import oracle
 from llaisys_amd.hostfmt import f32_to_bf16
+from llaisys_amd.libllaisys import LIB_LLAISYS
 from numerics import assert_exact, assert_linear_close
 from test_norm_linear_gpu import Case
 from test_linear_gpu import AMD, DTS, dev, int8_weights, linear, linear_w8a16, sample
@@ -74,6 +76,74 @@ def test_swiglu_epilogue_equals_separate_ops(rows, in_f, out_f, dt):
         want, _, h_want = c.composed()
         assert_exact(h, h_want, "residual")
         assert_exact(got, want, f"int8={int8}")
+
+
+def in_new_thread(body):
+    """body() in a thread of its own: its own scratch, not grown yet"""
+    result, errors = [], []
+
+    def run():
+        try:
+            result.append(body())
+        except BaseException as e:  # re-raised in the test thread
+            errors.append(e)
+
+    th = threading.Thread(target=run)
+    th.start()
+    th.join()
+    if errors:
+        raise errors[0]
+    return result[0]
+
+
+def test_scratch_grows_by_half_at_least():
+    """Prompts of a row more each find the scratch grown a few times, not at every one (a growth waits for
+    the device)."""
+    size = LIB_LLAISYS.llaisysTestWorkspaceBytes
+    size.restype = ctypes.c_size_t
+
+    def body():
+        x, w = dev(np.zeros((64, 8960), np.float16)), dev(np.zeros((1536, 8960), np.float16))
+        sizes = set()
+        for rows in range(17, 65):
+            L.Ops.linear(L.Tensor((rows, 1536), DTS["f16"], **AMD), x.slice(0, 0, rows), w)
+            sizes.add(size(0))
+        L.RuntimeAPI(L.DeviceType.AMD).device_synchronize()
+        return sizes
+
+    sizes = in_new_thread(body)
+    assert 1 < len(sizes) <= 5, sizes
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f32"])
+def test_split_k_is_the_same_in_a_graph(monkeypatch, dt):
+    """With the scratch a capture reserves by itself a linear splits as it does outside; with room for its
+    own partial sums but not for those of gate and up in one launch, neither that launch nor the
+    linear on one half splits."""
+    rng = np.random.default_rng(6)
+    rows, in_f, out_f = 64, 8960, 512
+    x, w = sample(rng, (rows, in_f), dt), sample(rng, (out_f, in_f), dt, 0.05)
+
+    def captured(reserve):
+        if reserve is None:
+            monkeypatch.delenv("LLAISYS_GRAPH_WORKSPACE_BYTES", raising=False)
+        else:
+            monkeypatch.setenv("LLAISYS_GRAPH_WORKSPACE_BYTES", str(reserve))
+        tx, tw, out = dev(x, DTS[dt]), dev(w, DTS[dt]), L.Tensor((rows, out_f), DTS[dt], **AMD)
+        graph = L.Graph.capture()
+        L.Ops.linear(out, tx, tw)
+        graph.end()
+        for _ in range(2):
+            graph.launch()
+            L.RuntimeAPI(L.DeviceType.AMD).device_synchronize()
+        return out.numpy()
+
+    eager = in_new_thread(lambda: linear(x, w, None, dt))
+    assert_exact(in_new_thread(lambda: captured(None)), eager, "default reserve")
+    unsplit = in_new_thread(lambda: captured(0))
+    assert not np.array_equal(unsplit, eager)  # a shape that splits, seen in its bits
+    own = 32 * rows * out_f * 4
+    assert_exact(in_new_thread(lambda: captured(own)), unsplit, "its own partial sums only")
 
 
 def test_split_k_under_capture_without_workspace(monkeypatch):
