@@ -26,6 +26,13 @@ void setSplits(Plan &p, const LinearCall &c, size_t want) {
     p.splits = int(ceilDiv(nk, p.per));
 }
 
+// setSplits for the 16-bit tiles, of stages of 64 k: the dense 192 x 256 tile takes the same ranges of K
+// in stages of 32
+void splitStages(Plan &p, const LinearCall &c, size_t want) {
+    setSplits(p, c, want);
+    if (p.tile == GemmTile::k192x256 && !c.scale) p.ks = 32, p.per *= 2;
+}
+
 // Splits that bring the blocks to `blocks`, each with at least `least` stages.  The outputs N are
 // counted once with swiglu too, so that it sums as the two separate linears do.
 void fillSplits(Plan &p, const LinearCall &c, size_t blocks, size_t least) {
@@ -61,8 +68,8 @@ struct TileTime {
 };
 constexpr TileTime kDense[] = {
     {GemmTile::k64x64, 64, 64, 3, {360, 450, 640}},      {GemmTile::k128x64, 128, 64, 3, {580, 700, 1100}},
-    {GemmTile::k96x128, 96, 128, 1, {700}},              {GemmTile::k128x128, 128, 128, 2, {800, 1300}},
-    {GemmTile::k192x128, 192, 128, 1, {950}},            {GemmTile::k192x256, 192, 256, 1, {1700}},
+    {GemmTile::k128x128, 128, 128, 2, {800, 1300}},      {GemmTile::k192x128, 192, 128, 1, {950}},
+    {GemmTile::k192x256, 192, 256, 1, {1700}},
 };
 constexpr TileTime kCodes[] = {
     {GemmTile::k64x64, 64, 64, 3, {450, 650, 770}},      {GemmTile::k128x64, 128, 64, 3, {650, 800, 1130}},
@@ -113,9 +120,7 @@ Plan plan16(const LinearCall &c) {
         for (const TileTime &t : kCodes) pick(t);
     else
         for (const TileTime &t : kDense) pick(t);
-    setSplits(p, c, splits);
-    // stages of 32 k: the same ranges of K
-    if (p.tile == GemmTile::k192x256 && !c.scale) p.ks = 32, p.per *= 2;
+    splitStages(p, c, splits);
     return p;
 }
 
@@ -151,10 +156,8 @@ bool gemmTakes(const LinearCall &c) {
 
 size_t gemmWorkspaceBytes(const LinearCall &c) { return planBytes(planOf(c), c); }
 
-void gemm(const LinearCall &c, void *ws, size_t ws_bytes, hipStream_t s) {
-    if (c.rows == 0 || c.N == 0) return;
-    Plan p = planOf(c);
-    if (planBytes(p, c) > ws_bytes) setSplits(p, c, 1);
+namespace {
+void launchPlan(const Plan &p, const LinearCall &c, void *ws, hipStream_t s) {
     const size_t es = c.dt == LLAISYS_DTYPE_F32 ? 4 : 2;
     GemmArgs a{};
     a.out = c.out;
@@ -176,6 +179,41 @@ void gemm(const LinearCall &c, void *ws, size_t ws_bytes, hipStream_t s) {
         gemmF16(p.tile, a, c.swiglu, s);
     else
         c.swiglu ? launchF32<true>(p, a, s) : launchF32<false>(p, a, s);
+}
+} // namespace
+
+void gemm(const LinearCall &c, void *ws, size_t ws_bytes, hipStream_t s) {
+    if (c.rows == 0 || c.N == 0) return;
+    Plan p = planOf(c);
+    if (planBytes(p, c) > ws_bytes) setSplits(p, c, 1);
+    launchPlan(p, c, ws, s);
+}
+
+extern "C" int llaisysTestLinearPlan(size_t rows, size_t K, size_t N, int int8, int swiglu, int dt, int plan[4]) {
+    static const float one = 1.0f;
+    const Plan p = planOf({nullptr, nullptr, nullptr, int8 ? &one : nullptr, nullptr, rows, K, N, swiglu != 0, llaisysDataType_t(dt)});
+    plan[0] = int(p.tile);
+    plan[1] = p.splits;
+    plan[2] = p.per;
+    plan[3] = p.ks;
+    return 0;
+}
+
+extern "C" int llaisysTestLinearTile(void *out, const void *x, const void *w, const float *scale, const void *bias, size_t rows,
+                                     size_t K, size_t N, int swiglu, int dt, int tile, size_t splits, void *ws, size_t ws_bytes) {
+    const LinearCall c{out, x, w, scale, bias, rows, K, N, swiglu != 0, llaisysDataType_t(dt)};
+    if (dt == LLAISYS_DTYPE_F32 || !gemmTakes(c) || splits == 0) return 0;
+    Plan p{GemmTile(tile), 0, 0, 0, 1, 0};
+    if (p.tile == GemmTile::k64x64Deep) p.ks = 128;
+    if (scale)
+        for (const TileTime &t : kCodes) p.ks = t.tile == p.tile ? 64 : p.ks;
+    else
+        for (const TileTime &t : kDense) p.ks = t.tile == p.tile ? 64 : p.ks;
+    if (p.ks == 0) return 0;
+    splitStages(p, c, splits);
+    if (planBytes(p, c) > ws_bytes) return 0;
+    launchPlan(p, c, ws, nullptr);
+    return hipGetLastError() == hipSuccess && hipDeviceSynchronize() == hipSuccess ? p.splits : 0;
 }
 
 } // namespace llaisys::kernels

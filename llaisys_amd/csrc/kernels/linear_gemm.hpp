@@ -12,6 +12,13 @@ bool gemmTakes(const LinearCall &c);
 size_t gemmWorkspaceBytes(const LinearCall &c);
 void gemm(const LinearCall &c, void *ws, size_t ws_bytes, hipStream_t s);
 
+// For the tests.  The plan of a call: tile, splits, stages per split, k per stage (no GPU needed).
+extern "C" int llaisysTestLinearPlan(size_t rows, size_t K, size_t N, int int8, int swiglu, int dt, int plan[4]);
+// A 16-bit call on the tile and split given, on the default stream and waited for, with `ws` for its
+// partial sums: the splits it ran with, 0 for a tile or call that there is none for.
+extern "C" int llaisysTestLinearTile(void *out, const void *x, const void *w, const float *scale, const void *bias, size_t rows,
+                                     size_t K, size_t N, int swiglu, int dt, int tile, size_t splits, void *ws, size_t ws_bytes);
+
 // ---- between linear_gemm.hip and the kernels ---------------------------------------------------
 
 struct GemmArgs {
@@ -28,7 +35,7 @@ struct GemmArgs {
 
 // Tile shapes of the 16-bit types, weight rows x activation rows (64x64Deep: stages of 128 k shared
 // by two waves per tile quarter).
-enum class GemmTile { k64x64Deep, k64x64, k128x64, k96x128, k128x128, k192x128, k256x128, k192x256 };
+enum class GemmTile { k64x64Deep, k64x64, k128x64, k128x128, k192x128, k256x128, k192x256 };
 
 void gemmBf16(GemmTile t, const GemmArgs &a, bool swiglu, hipStream_t s);
 void gemmF16(GemmTile t, const GemmArgs &a, bool swiglu, hipStream_t s);

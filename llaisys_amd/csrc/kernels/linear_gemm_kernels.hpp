@@ -158,7 +158,7 @@ __global__ void __launch_bounds__(NWW *NWX *NWK * 64)
     // is a compile-time promise that kt is not the last stage: the loop over all but the last S
     // stages then has no branch around its loads and one constant wait, and the compiler places the
     // loads among the LDS reads and MFMAs (2048 rows of gate / up / swiglu 129.8 -> 127.1 us, one
-    // [8960, 1536] 83.2 -> 79.4 in tiles of 192 x 256, 79.8 -> 79.0 in 192 x 128; 96 x 128 -8%).
+    // [8960, 1536] 83.2 -> 79.4 in tiles of 192 x 256, 79.8 -> 79.0 in 192 x 128).
     const auto issue = [&](int kt, auto steady) {
         char *dst = lds + (kt % S) * kStageB;
         if (!steady && tail && kt == nk - 1) {
@@ -482,7 +482,6 @@ void launch16(GemmTile t, const GemmArgs &a, hipStream_t s) {
         case GemmTile::k64x64Deep: launchTile<T, false, kSw, 64, 64, 2, 1, 2, 128, 2>(a, s); break;
         case GemmTile::k64x64: launchTile<T, false, kSw, 64, 64, 2, 2, 1, 64, 3>(a, s); break;
         case GemmTile::k128x64: launchTile<T, false, kSw, 128, 64, 2, 2, 1, 64, 2>(a, s); break;
-        case GemmTile::k96x128: launchTile<T, false, kSw, 96, 128, 1, 4, 1, 64, 4>(a, s); break;
         case GemmTile::k128x128: launchTile<T, false, kSw, 128, 128, 2, 2, 1, 64, 2>(a, s); break;
         case GemmTile::k192x128: launchTile<T, false, kSw, 192, 128, 2, 4, 1, 64, 3, true>(a, s); break;
         default: launchTile<T, false, kSw, 192, 256, 2, 4, 1, 32, 5, true>(a, s); break;

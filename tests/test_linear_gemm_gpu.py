@@ -33,10 +33,10 @@ def test_f32_tiles(shape):
     assert_exact(linear(x, w, b, "f32"), got, "repeat")
 
 
-# rows, in_features, out_features of the 16-bit tiles: the 64-row tile with its deep stages (first and
-# last row count, K of one chunk pair, a ragged last stage, split), then the tiles that the expected
-# launch time picks as the rows grow (64 x 64, 128 x 64, 96 x 128, 128 x 128, 192 x 128, 256 x 128,
-# 192 x 256), each with ragged channels or rows, one stage or a ragged last one, and split
+# rows, in_features, out_features through the public calls: the 64-row tile with its deep stages (first and
+# last row count, K of one chunk pair, a ragged last stage, split), then what the expected launch time
+# picks as the rows grow, mostly 64 x 64 tiles, split and not, and larger ones over a few stages, with
+# ragged channels or rows (test_each_tile has every tile over many stages)
 EDGES = [(17, 16, 64), (64, 144, 63), (37, 1552, 130), (64, 8960, 66), (65, 16, 65), (96, 208, 300), (128, 8960, 192),
          (161, 1552, 2000), (300, 4112, 140), (300, 64, 9002), (800, 80, 9001), (1024, 2064, 770), (1500, 96, 1531),
          (2047, 48, 9003), (3999, 112, 1540), (2048, 64, 18000)]
@@ -76,6 +76,58 @@ def test_swiglu_epilogue_equals_separate_ops(rows, in_f, out_f, dt):
         want, _, h_want = c.composed()
         assert_exact(h, h_want, "residual")
         assert_exact(got, want, f"int8={int8}")
+
+
+# GemmTile: weight rows, activation rows and k per stage; the 256 x 128 tile is for INT8 weights only, and
+# dense weights take 192 x 256 in stages of 32
+TILES = {"64x64deep": (0, 64, 64, 128), "64x64": (1, 64, 64, 64), "128x64": (2, 128, 64, 64), "128x128": (3, 128, 128, 64),
+         "192x128": (4, 192, 128, 64), "256x128": (5, 256, 128, 64), "192x256": (6, 192, 256, 64)}
+# stages of the tile's k, what the last one lacks, splits: fewer stages than the ring of LDS tiles holds (2 to
+# 5), as many, one more, odd and even counts beyond; ranges of K that start past 0, the last one short
+STAGES = [(1, 48, 1), (2, 0, 1), (3, 16, 1), (4, 0, 1), (5, 32, 1), (8, 0, 1), (9, 16, 1), (4, 16, 2), (9, 0, 2), (19, 48, 3)]
+
+
+def on_tile(tile, x, w, scale, bias, dt, swiglu, splits, ws):
+    """The rows of x through `tile`, K in `splits` ranges (llaisysTestLinearTile)."""
+    n = w.shape[0] // 2 if swiglu else w.shape[0]
+    tx, tw, out = dev(x, DTS[dt]), dev(w, None if scale is not None else DTS[dt]), L.Tensor((x.shape[0], n), DTS[dt], **AMD)
+    ts, tb = None if scale is None else dev(scale), None if bias is None else dev(bias, DTS[dt])
+    ptr = lambda t: ctypes.c_void_p(None if t is None else t.data_ptr())
+    got = LIB_LLAISYS.llaisysTestLinearTile(ptr(out), ptr(tx), ptr(tw), ptr(ts), ptr(tb), *(ctypes.c_size_t(v) for v in (*x.shape, n)),
+                                            int(swiglu), int(DTS[dt]), tile, ctypes.c_size_t(splits), ptr(ws),
+                                            ctypes.c_size_t(ws.shape()[0] * 4))
+    assert got == splits, (tile, got)
+    return out.numpy()
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("int8", [False, True], ids=["dense", "int8"])
+@pytest.mark.parametrize("name", TILES)
+def test_each_tile(name, int8, dt):
+    """Every tile against the oracle, and its swiglu epilogue (in the tile, or in the sum over splits) bit
+    for bit against the two halves on the same tile."""
+    tile, bw, bx, ks = TILES[name]
+    if name == "256x128" and not int8:
+        return
+    rng = np.random.default_rng(zlib.crc32(repr((name, int8, dt)).encode()))
+    ws = L.Tensor((8 << 20,), DTS["f32"], **AMD)
+    for stages, lacks, splits in STAGES:
+        rows, n, k = bx + int(rng.integers(1, 40)), bw + 2 * int(rng.integers(1, 40)), stages * ks - lacks
+        x, b = sample(rng, (rows, k), dt), sample(rng, (2 * n,), dt)
+        what = f"{name} {rows}x{k}x{n} / {splits}"
+        if int8:
+            w, scale = int8_weights(rng, 2 * n, k)
+            gate, up = ((w[h], scale[h], b[h]) for h in (slice(n), slice(n, None)))
+            want = oracle.linear_w8a16(x, *gate)
+        else:
+            w, scale = sample(rng, (2 * n, k), dt, 0.05), None
+            gate, up = ((w[h], None, b[h]) for h in (slice(n), slice(n, None)))
+            want = oracle.linear(x, gate[0], gate[2])
+        y = [on_tile(tile, x, *half, dt, False, splits, ws) for half in (gate, up)]
+        assert_linear_close(y[0], want, x, gate[0], what, **({"w_scale": gate[1]} if int8 else {}))
+        out = L.Tensor((rows, n), DTS[dt], **AMD)
+        L.Ops.swiglu(out, dev(y[0], DTS[dt]), dev(y[1], DTS[dt]))
+        assert_exact(on_tile(tile, x, w, scale, b, dt, True, splits, ws), out.numpy(), "swiglu " + what)
 
 
 def in_new_thread(body):
