@@ -199,6 +199,7 @@ __global__ void __launch_bounds__(NWW *NWX *NWK * 64)
         // complete in LDS one stage before its MFMAs.
         static_assert(NWK == 1 && kE == 2 && S >= 3, "pipelined tiles");
         constexpr int kPairs = XC / 4, CW = kInt8 ? 1 : 2; // chunks of a weight row per pair
+        constexpr int kReads = TW * CW + 2 * TX, kMfmas = 2 * TW * TX, kPaired = kReads < kMfmas ? kReads : kMfmas;
         struct Ops {
             v4u w[TW][CW], x[TX][2];
         };
@@ -240,13 +241,14 @@ __global__ void __launch_bounds__(NWW *NWX *NWK * 64)
                 else
                     fetch(n, kt + 1, 0); // past the last stage: read, not used
                 multiply(c);
-                // one LDS read behind each of the first MFMAs
+                // one LDS read behind each of the first MFMAs (behind the last one what is left of them)
 #pragma unroll
-                for (int r = 0; r < TW * CW + 2 * TX; ++r) {
+                for (int r = 0; r < kPaired; ++r) {
                     __builtin_amdgcn_sched_group_barrier(0x008, 1, 0); // MFMA
                     __builtin_amdgcn_sched_group_barrier(0x100, 1, 0); // LDS read
                 }
-                __builtin_amdgcn_sched_group_barrier(0x008, 2 * TW * TX - (TW * CW + 2 * TX), 0);
+                if constexpr (kReads > kPaired) __builtin_amdgcn_sched_group_barrier(0x100, kReads - kPaired, 0);
+                if constexpr (kMfmas > kPaired) __builtin_amdgcn_sched_group_barrier(0x008, kMfmas - kPaired, 0);
             }
         };
         Ops o0, o1;
