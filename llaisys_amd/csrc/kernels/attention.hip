@@ -398,7 +398,7 @@ __global__ void __launch_bounds__(kWave)
         for (int e = lane; e < dv; e += kWave) acc[e] = acc[e] * corr + p * vval(t, e);
         m = mx;
     }
-    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    const float inv = l == 0.0f ? 0.0f : 1.0f / l; // (NaN for a NaN score)
     for (int e = lane; e < dv; e += kWave) Fmt<T>::put(a.out, ih * dv + e, acc[e] * inv);
 }
 

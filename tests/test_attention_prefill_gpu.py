@@ -129,9 +129,9 @@ def test_non_finite_v_reaches_only_queries_that_see_it(value, shape, dt, d, int8
 
 
 # seq, total, nh, nkvh, d: prefill in one piece and with the keys split over few and many blocks, decode
-# in one piece and split, head_dim 64
+# in one piece and split, head_dim 64, and one that the scalar kernel takes
 BAD_SCORES = [(40, 40, 4, 2, 128), (33, 1100, 3, 1, 64), (16, 9000, 2, 1, 128), (5, 40, 4, 2, 128), (2, 3000, 12, 2, 128),
-              (3, 700, 4, 2, 64)]
+              (3, 700, 4, 2, 64), (7, 40, 4, 2, 24)]
 
 
 @pytest.mark.parametrize("dt", ["bf16", "f16", "f32"])
