@@ -440,16 +440,19 @@ __device__ __forceinline__ v4u codesToBf16(const v4u &raw, float sc) {
 // 16 g + 8 a + 4 h + b of K is key 16 g + 8 h + 4 a + b, so lane half h ends with the scores of keys
 // 16 g + 8 h + 0 .. 7 of its query -- the 8 consecutive k of the P V product's B operand -- and the
 // softmax needs one exchange between the two lanes of a query.  P enters as two 16-bit parts (hi +
-// lo: 2^-17 relative in bf16, 2^-22 in f16), so the output keeps f32 accuracy; in f16 the weights
-// carry a factor 2^8, which keeps the parts of small weights normal numbers and cancels in O / l.
+// lo: 2^-17 relative in bf16, 2^-22 in f16), which is less than the f32 weights of the vector kernel:
+// over 12 to 32 heads and 16 to 1500 keys the error against 64 bits is the vector kernel's to five
+// digits in bf16 (4 to 15 in 10000 outputs are not the exact value's rounding, 1 to 4 there) and within
+// 0.5% in f16.  In f16 the weights carry a factor 2^8, which keeps the low parts of weights down to 2^-11
+// normal numbers and cancels in O / l.
 //
 // K and V tiles move HBM -> LDS with global_load_lds_dwordx4 (1 KB per instruction, two stages, the
 // next step's loads in flight during this one's math).  V stays row-major; its transposed operand
 // is two ds_read_b64_tr_b16: within 16 lanes, lane j's element e is element j % 4 of the 8 bytes
 // that lane 4 e + j / 4 addresses.  Rows cannot be padded (the load fills LDS contiguously), so the
 // 16-byte chunks of a row are XOR-swizzled: K so that 16 rows' reads of one chunk touch all banks,
-// V so that the 64-byte pieces of 4 rows do.  An INT8 cache is dequantized into the workspace when
-// it fits, else its codes are converted on their way into LDS (the same operands, the same bits).
+// V so that the 64-byte pieces of 4 rows do.  The codes of an INT8 cache are converted on their way into
+// LDS, or the cache is dequantized into the workspace first (planPrefill; the same operands, the same bits).
 // Keys past the cache read row 0 and weigh 0, as masked keys do; what a non-finite V element of
 // such a row leaves in the sums is replaced at the end (visibleSum).
 //
@@ -459,8 +462,8 @@ __device__ __forceinline__ v4u codesToBf16(const v4u &raw, float sc) {
 // per wave), or four waves on a SIMD, came to the same 3.8 us per 256 keys, and running one unit half a
 // step behind the other spilled registers.
 // 2048 queries, 12 / 2 heads, bf16: 44.9 us with 16-query tiles and one wave per q head on 16 x 16
-// x 32 MFMAs (1 KB of LDS read per 16 MFMA cycles, CUs with early queries idle) -> 34.9 us; f16, 300
-// queries over 1500 INT8 keys: 479 us on the vector kernel -> 23 us.
+// x 32 MFMAs (1 KB of LDS read per 16 MFMA cycles, CUs with early queries idle) -> 36.4 us; f16, 300
+// queries over 1500 INT8 keys: 479 us on the vector kernel -> 25.5 us.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -1434,11 +1437,11 @@ double dequantizeUs(size_t el) {
 //    chunks of at least 4 steps (512 keys): 16 queries over 32768 keys would otherwise be 256 steps in
 //    each of 6 blocks.
 //  - Its block costs about 4 us beside its steps, so calls of few steps and of less than two rounds of
-//    small blocks run faster on attnPrefill16 (bf16, 128; 100 queries, 32 / 8 heads 8.4 -> 6.5 us) or
-//    attnGroup (16 queries, 16 / 16 heads of 64, bf16 5.7 -> 4.0 us).
+//    small blocks run faster on attnPrefill16 (bf16, 128; 100 queries, 32 / 8 heads 8.3 -> 6.2 us) or
+//    attnGroup (16 queries, 16 / 16 heads of 64, bf16 6.2 -> 4.7 us).
 //  - attnPrefill converts a bf16 INT8 cache in the kernel until the query blocks that convert a tile again
 //    cost more than one launch that dequantizes it (16 / 16 heads of 128, 64 queries over 1264 keys 28.8 ->
-//    21.0 us; from about 3000 queries the other way round).  f16 codes cost five times as much.
+//    21.6 us; from about 3000 queries the other way round).  f16 codes cost five times as much.
 bool planPrefill(Prefill &p, const AttnArgs &a, int d, int dv, bool int8, llaisysDataType_t dt) {
     const bool bf16 = dt == LLAISYS_DTYPE_BF16;
     if ((!bf16 && dt != LLAISYS_DTYPE_F16) || !vecShape(a, d, dv, int8)) return false;

@@ -148,7 +148,8 @@ __global__ void __launch_bounds__(NW * kWave)
 // gate/up + swiglu [2 x 8960, 1536] 9.99 -> 10.46 us INT8, 16 waves 12.67 us).
 // Channels per wave: 2 where one each would take more waves than the chip holds (256 CUs x 32), so that
 // no second round of blocks forms the row again and x is unpacked for twice the rows: INT8 [17920,
-// 1536] 11.83 -> 10.09 us, gate/up + swiglu [2 x 8960, 1536] 10.34 -> 9.97 us; bf16 [17920, 1536] 12.57 ->
+// 1536] 11.83 -> 10.09 us, gate/up + swiglu [2 x 8960, 1536] 10.34 -> 9.97 us (launched over
+// and over; a decode layer that holds it takes the same 35.8 us with either); bf16 [17920, 1536] 12.57 ->
 // 11.75 us.  16-bit gate/up rows keep one (11.93 -> 12.54 us with two), and 4 channels lose for INT8
 // gate/up (12.44 us).
 constexpr int kWavesAtOnce = 256 * 32;

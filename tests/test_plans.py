@@ -46,8 +46,8 @@ SHORT = [((16, 16, 16, 16, 128, "bf16"), K16, 1), ((100, 100, 32, 8, 128, "bf16"
 
 @pytest.mark.parametrize("shape, kernel, heads", SHORT)
 def test_short_prefills_take_the_faster_kernel(shape, kernel, heads):
-    """Measured on both sides of the line; 100 queries of 32 / 8 heads take 8.4 us in blocks of 32 queries and
-    6.5 us in blocks of 16."""
+    """Measured on both sides of the line; 100 queries of 32 / 8 heads take 8.3 us in blocks of 32 queries and
+    6.2 us in blocks of 16."""
     route = attention_route(*shape[:5], False, shape[5])
     assert (route[0], route[4]) == (kernel, heads)
 
